@@ -1,9 +1,11 @@
 // Prefill kernels for gfx950: MFMA BF16 GEMM (plain or .p12 weights) with fused epilogues,
 // row RMSNorm / residual kernels and the K/V cache writer.
 //
-//   gemm_dma_kernel Y[t][m] = sum_k X[t][k] W[m][k] for plain BF16 weights: 256x128 or 128x128
-//                   tiles, BK 64, operands loaded straight into three swizzled LDS stages,
+//   gemm_dma_kernel Y[t][m] = sum_k X[t][k] W[m][k] for plain BF16 weights and many tokens:
+//                   large tiles, operands loaded straight into swizzled LDS stages,
 //                   v_mfma_f32_32x32x16_bf16, XCD-grouped tiles.
+//   gemm_small_kernel  the same for fewer tokens: tiles of 16x16 blocks down to one block, so
+//                   that short prompts fill the chip too.
 //   gemm_kernel     the same product for .p12 weights, expanded in registers on the way to a
 //                   double-buffered LDS tile.  Both replace `matrix` (Kernels.metal:149-200)
 //                   for the projections and `swiglu` (Kernels.metal:202-210) as an epilogue.
@@ -267,21 +269,21 @@ __device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t v, void* lds,
 
 // Plain-weight GEMM whose operand tiles go from memory straight into LDS (buffer loads with
 // the LDS destination): no staging registers and no LDS store instructions.  NS LDS stages of
-// KD K values each, NS - 1 stages in flight.  A stage holds BT activation rows then BW weight
-// rows of KD * 2 bytes; the 16-byte chunk c of row R sits in slot c ^ ((R >> SH) & (CPR - 1))
-// (SH = 1 for 128-byte rows, 2 for 64-byte rows), which spreads both the loads' row segments
-// and the operand reads' 16-row columns over all banks.  Each wave loads Q 1 KB blocks per
-// stage.  Waves synchronise with a bare s_barrier after waiting for their own stage loads and
-// LDS reads, so the later stages stay in flight across the barrier.
-template <int EPI, int BT, int BW, int WT, int NT, int KD, int NS>
+// 64 K values each, NS - 1 stages in flight.  A stage holds BT activation rows then BW weight
+// rows of 128 bytes; the 16-byte chunk c of row R sits in slot c ^ ((R >> 1) & 7), which
+// spreads both the loads' row segments and the operand reads' 16-row columns over all banks.
+// Each wave loads Q 1 KB blocks per stage.  Waves synchronise with a bare s_barrier after
+// waiting for their own stage loads and LDS reads, so the later stages stay in flight across
+// the barrier.
+template <int EPI, int BT, int BW, int WT, int NT, int NS>
 __global__ __launch_bounds__(NT) void gemm_dma_kernel(const GemmParams p, int col_tiles, int row_tiles) {
+    constexpr int KD = 64, SH = 1;
     constexpr int NW = NT / 64, WW = NW / WT, TT = BT / WT / 32, TW = BW / WW / 32;
-    constexpr int ROWB = KD * 2, CPR = ROWB / 16, RPI = 1024 / ROWB, SH = ROWB == 128 ? 1 : 2;
+    constexpr int ROWB = KD * 2, CPR = ROWB / 16, RPI = 1024 / ROWB;
     constexpr int ROWS = BT + BW, STAGE = ROWS * ROWB, Q = ROWS / RPI / NW;
-    static_assert(KD == 64 || KD == 32, "stage depth");
     static_assert(ROWS % (RPI * NW) == 0 && BT % 16 == 0, "stage blocks per wave");
     static_assert(EPI != GEMM_SWIGLU || TW % 2 == 0, "SwiGLU pairs gate and up tiles inside a wave");
-    static_assert(NS >= 3, "at least two stages in flight");
+    static_assert(NS == 3 || NS == 4, "two or three stages in flight");
     // one array per stage: the compiler then tells the stages apart and waits for the loads
     // into a stage only before reading that stage (one shared array would make every read
     // wait for every load in flight)
@@ -289,17 +291,12 @@ __global__ __launch_bounds__(NT) void gemm_dma_kernel(const GemmParams p, int co
     __shared__ __align__(1024) uint8_t S1[STAGE];
     __shared__ __align__(1024) uint8_t S2[STAGE];
     __shared__ __align__(1024) uint8_t S3[NS > 3 ? STAGE : 16];
-    __shared__ __align__(1024) uint8_t S4[NS > 4 ? STAGE : 16];
-    __shared__ __align__(1024) uint8_t S5[NS > 5 ? STAGE : 16];
-    static_assert(NS <= 6, "at most six stages");
     auto stage_of = [&](auto idx) -> uint8_t* {
         constexpr int i = decltype(idx)::value;
         if constexpr (i == 0) return S0;
         else if constexpr (i == 1) return S1;
         else if constexpr (i == 2) return S2;
-        else if constexpr (i == 3) return S3;
-        else if constexpr (i == 4) return S4;
-        else return S5;
+        else return S3;
     };
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (scalar)
@@ -390,6 +387,191 @@ __global__ __launch_bounds__(NT) void gemm_dma_kernel(const GemmParams p, int co
     // in flight: the workgroup's LDS may go to the next workgroup on this CU.
     wait_vmcnt<0>();
     gemm_epilogue<EPI, TT, TW>(p, acc, t0 + wt * TT * 32, n0, ww, lane);
+}
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+// A buffer view as its four resource words, and load_to_lds (16 bytes per lane to `lds` + 16 lane)
+// as a statement the compiler does not track.  Of loads it tracks, it waits for every one in
+// flight before an LDS read that it cannot tell from their destinations, which serialises most
+// stage layouts (16 tokens x 6144: 28 us instead of 12); here the kernel's own vmcnt waits order
+// loads and reads.  No register is written, so nothing in flight can clobber one.  (s_nop: the
+// wait state between a write of M0 and a load into LDS.)
+__device__ __forceinline__ u32x4_t view_words(const void* base, uint32_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(base);
+    return u32x4_t{uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(a)))),
+                   uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(a >> 32) & 0xffffu))),
+                   uint32_t(__builtin_amdgcn_readfirstlane(int(bytes))), 0x00020000u};
+}
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+    return uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p));
+}
+__device__ __forceinline__ void load_to_lds_untracked(const u32x4_t view, uint32_t lds, uint32_t off) {
+    __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     :
+                     : "s"(__builtin_amdgcn_readfirstlane(int(lds))), "v"(off), "s"(view)
+                     : "m0", "memory");
+}
+
+// The same product on small tiles, for calls whose 32-row tiles would leave most CUs idle
+// (up to about 1,000 tokens): BT tokens x BM weight rows as 16x16 blocks of
+// v_mfma_f32_16x16x32_bf16, whose result equals two v_mfma_f32_32x32x16_bf16 steps bit for bit
+// (both fold K in groups of eight in ascending order), at half the latency per K.  A stage is H
+// slabs of 64 K values, each [BT activation rows | BM weight rows] of 128 bytes loaded and
+// swizzled as in gemm_dma_kernel; NS stages in a ring, NS - 1 in flight.  WT x WM waves own the
+// outputs ((BT / WT) x (BM / WM) each); every wave of the workgroup loads.  Weights are the MFMA's
+// row operand, so a lane holds four consecutive outputs of one token.
+template <int EPI, int BT, int BM, int WT, int WM, int NT, int H, int NS>
+__global__ __launch_bounds__(NT) void gemm_small_kernel(const GemmParams p, int col_tiles, int row_tiles, int wide) {
+    constexpr int NW = NT / 64, TT = BT / WT / 16, TM = BM / WM / 16;
+    constexpr int ROWS = BT + BM, SLAB = ROWS * 128, STAGE = H * SLAB;
+    // 1 KB blocks (eight rows) of a stage: XB of activations, WB of weights, dealt to the waves
+    // apart, so that no load's source depends on the wave (where the blocks do not divide, the
+    // last waves load some twice)
+    constexpr int XB = H * BT / 8, WB = H * BM / 8, QX = (XB + NW - 1) / NW, QW = (WB + NW - 1) / NW, Q = QX + QW;
+    static_assert(BT % 16 == 0 && BM % 16 == 0 && WT * WM <= NW, "tile");
+    static_assert(TT >= 1 && TM >= 1 && TT * WT * 16 == BT && TM * WM * 16 == BM, "wave tile");
+    static_assert(EPI != GEMM_SWIGLU || TM % 2 == 0, "SwiGLU pairs gate and up blocks inside a wave");
+    static_assert(NS >= 2 && (NS - 2) * Q < 64, "loads in flight");
+    __shared__ __align__(1024) uint8_t S[NS * STAGE];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tiles = col_tiles * row_tiles;
+    const int per = (tiles + 7) / 8;
+    const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (tile >= tiles) return;
+    const int ct = tile / row_tiles, rt = tile % row_tiles;
+    const int t0 = rt * BT;
+    const int n0 = ct * (EPI == GEMM_SWIGLU ? BM / 2 : BM);
+    const uint32_t K = uint32_t(p.k);
+    const int nk = p.k / (64 * H);
+    const u32x4_t xv = view_words(p.x, uint32_t(p.tokens) * K * 2u), wv = view_words(p.w, uint32_t(p.m) * K * 2u);
+    const uint32_t lds = lds_address(S);
+
+    // this lane's source offset (stage 0) for each of the wave's blocks
+    uint32_t xoff[QX], woff[QW], xdst[QX], wdst[QW];
+#pragma unroll
+    for (int q = 0; q < QX; ++q) {
+        const int id = (wave * QX + q) % XB, h = id / (BT / 8), R = id % (BT / 8) * 8 + (lane >> 3);
+        const uint32_t c = uint32_t((lane & 7) ^ ((R >> 1) & 7));
+        xoff[q] = (uint32_t(t0 + R) * K + uint32_t(h) * 64u + c * 8) * 2u;
+        xdst[q] = uint32_t(h * SLAB + id % (BT / 8) * 1024);
+    }
+#pragma unroll
+    for (int q = 0; q < QW; ++q) {
+        const int id = (wave * QW + q) % WB, h = id / (BM / 8), r = id % (BM / 8) * 8 + (lane >> 3);
+        const uint32_t c = uint32_t((lane & 7) ^ (((BT + r) >> 1) & 7));
+        uint32_t row;
+        if constexpr (EPI == GEMM_SWIGLU)  // 16 gate rows, then their 16 up rows
+            row = uint32_t(((r >> 4) & 1 ? INTER : 0) + n0 + (r >> 5) * 16 + (r & 15));
+        else row = uint32_t(n0 + r);
+        woff[q] = (row * K + uint32_t(h) * 64u + c * 8) * 2u;
+        wdst[q] = uint32_t(h * SLAB + BT * 128 + id % (BM / 8) * 1024);
+    }
+    auto issue = [&](uint32_t stage, int kt) {  // stage: its byte offset in S
+        const uint32_t kill = kt < nk ? 0u : OOB_OFFSET;
+        const uint32_t kb = uint32_t(kt) * (H * 128u);
+#pragma unroll
+        for (int q = 0; q < QX; ++q) load_to_lds_untracked(xv, lds + stage + xdst[q], (xoff[q] + kb) | kill);
+#pragma unroll
+        for (int q = 0; q < QW; ++q) load_to_lds_untracked(wv, lds + stage + wdst[q], (woff[q] + kb) | kill);
+    };
+    const bool computes = WT * WM == NW || wave < WT * WM;
+    const int wt = wave / WM, wm = wave % WM;
+    floatx4 acc[TM][TT];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    auto compute = [&](const uint8_t* stage) {
+#pragma unroll
+        for (int s = 0; s < 2 * H; ++s) {
+            const uint8_t* slab = stage + (s >> 1) * SLAB;
+            const int c = (s & 1) * 4 + (lane >> 4), r = lane & 15;
+            bf16x8 a[TM], b[TT];
+#pragma unroll
+            for (int j = 0; j < TT; ++j) {
+                const int R = (wt * TT + j) * 16 + r;
+                b[j] = as_bf16x8(*reinterpret_cast<const uint4*>(slab + R * 128 + ((c ^ ((R >> 1) & 7)) << 4)));
+            }
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                const int R = BT + (wm * TM + i) * 16 + r;
+                a[i] = as_bf16x8(*reinterpret_cast<const uint4*>(slab + R * 128 + ((c ^ ((R >> 1) & 7)) << 4)));
+            }
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TT; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+    };
+    // the waits of gemm_dma_kernel: own loads of this stage and own LDS reads of the last done,
+    // then the barrier; the stage before is then free
+    for (int b = 0; b < NS - 1; ++b) issue(uint32_t(b) * STAGE, b);
+    uint32_t cur = 0, freed = (NS - 1) * STAGE;
+    for (int kt = 0; kt < nk; ++kt) {
+        __asm__ volatile("" ::: "memory");
+        wait_vmcnt_lds<(NS - 2) * Q>();
+        __builtin_amdgcn_s_barrier();
+        __asm__ volatile("" ::: "memory");
+        issue(freed, kt + NS - 1);
+        if (computes) compute(S + cur);
+        freed = cur;
+        cur = cur + STAGE == NS * STAGE ? 0u : cur + STAGE;
+    }
+    wait_vmcnt<0>();  // no wave ends with a load into LDS in flight
+    if (!computes) return;
+
+    // Element r of a block is weight row 4 (lane / 16) + r, token lane % 16.  `wide`: the four
+    // outputs of a lane are stored together (m a multiple of four, y aligned to four outputs).
+    const uint32_t M = uint32_t(p.m);
+    const uint32_t cols = EPI == GEMM_SWIGLU ? uint32_t(INTER) : M;
+    constexpr uint32_t ES = EPI == GEMM_SWIGLU || EPI == GEMM_BF16 ? 2u : 4u;
+    const __amdgpu_buffer_rsrc_t yv =
+        buffer_view(ES == 2u ? static_cast<const void*>(p.y16) : static_cast<const void*>(p.y), uint32_t(p.tokens) * cols * ES);
+#pragma unroll
+    for (int j = 0; j < TT; ++j) {
+        const uint32_t t = uint32_t(t0 + (wt * TT + j) * 16 + (lane & 15));
+#pragma unroll
+        for (int i = 0; i < TM; i += EPI == GEMM_SWIGLU ? 2 : 1) {
+            const uint32_t m = uint32_t(n0 + (EPI == GEMM_SWIGLU ? (wm * TM + i) >> 1 : wm * TM + i) * 16 + (lane >> 4) * 4);
+            uint32_t w[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if constexpr (EPI == GEMM_SWIGLU) {  // as gemm_epilogue
+                    const float gt = roundbf(acc[i][j][r]);
+                    const float up = roundbf(acc[i + 1][j][r]);
+                    const float silu = gt / (1.0f + exp_det(-gt));
+                    w[r] = bits(roundbf(silu) * up);
+                } else if constexpr (EPI == GEMM_BF16) {
+                    w[r] = bits(acc[i][j][r]);
+                } else if constexpr (EPI == GEMM_F32) {
+                    w[r] = __float_as_uint(roundbf(acc[i][j][r]));
+                } else {
+                    w[r] = __float_as_uint(acc[i][j][r]);
+                }
+            }
+            const uint32_t e = t * cols + m;
+            if (wide) {
+                const uint32_t off = m < cols ? e * ES : OOB_OFFSET;
+                if constexpr (ES == 2u) {
+                    const u32x2_t v = {(w[0] & 0xffffu) | (w[1] << 16), (w[2] & 0xffffu) | (w[3] << 16)};
+                    __builtin_amdgcn_raw_buffer_store_b64(v, yv, off, 0, 0);
+                } else {
+                    const u32x4_t v = {w[0], w[1], w[2], w[3]};
+                    __builtin_amdgcn_raw_buffer_store_b128(v, yv, off, 0, 0);
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const uint32_t off = m + uint32_t(r) < cols ? (e + uint32_t(r)) * ES : OOB_OFFSET;
+                    if constexpr (ES == 2u) buffer_store2(yv, off, uint16_t(w[r]));
+                    else buffer_store4(yv, off, w[r]);
+                }
+            }
+        }
+    }
 }
 
 // ------------------------------------------------------------------------------ norms
@@ -1077,20 +1259,72 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_ranked_kernel(const Flas
     flash_prefill<QSA, DIRECT>(p, int(item >> 2), int(item & 3u));
 }
 
-template <int BT, int BW, int WT, int NT, int KD, int NS>
+template <int BT, int BW, int WT, int NT, int NS>
 void launch_gemm_dma(GemmEpilogue epi, const GemmParams& p, hipStream_t s) {
     const int cols = epi == GEMM_SWIGLU ? INTER / (BW / 2) : (p.m + BW - 1) / BW;
     const int rows = (p.tokens + BT - 1) / BT;
     const int per = (cols * rows + 7) / 8;
     const dim3 grid(8 * per), block(NT);
-#define PLAMO_GEMM(EP) hipLaunchKernelGGL((gemm_dma_kernel<EP, BT, BW, WT, NT, KD, NS>), grid, block, 0, s, p, cols, rows)
+#define PLAMO_GEMM(EP) hipLaunchKernelGGL((gemm_dma_kernel<EP, BT, BW, WT, NT, NS>), grid, block, 0, s, p, cols, rows)
     constexpr int TW = BW / (NT / 64 / WT) / 32;  // 32-column blocks per wave
+    if constexpr (TW % 2 == 0) {  // gate and up blocks pair inside a wave: the SwiGLU tile
+        PLAMO_GEMM(GEMM_SWIGLU);
+    } else {
+        if (epi == GEMM_F32) PLAMO_GEMM(GEMM_F32);
+        else if (epi == GEMM_BF16) PLAMO_GEMM(GEMM_BF16);
+        else PLAMO_GEMM(GEMM_RAW);
+    }
+#undef PLAMO_GEMM
+}
+
+template <int BT, int BM, int WT, int WM, int NT, int H, int NS>
+void launch_gemm_small(GemmEpilogue epi, const GemmParams& p, hipStream_t s) {
+    const int cols = epi == GEMM_SWIGLU ? INTER / (BM / 2) : (p.m + BM - 1) / BM;
+    const int rows = (p.tokens + BT - 1) / BT;
+    const int per = (cols * rows + 7) / 8;
+    const dim3 grid(8 * per), block(NT);
+    // four outputs per store where every row of y starts on such a boundary; the same check
+    // covers y itself, which may be a view with only its elements' alignment
+    const uintptr_t y = epi == GEMM_BF16 ? reinterpret_cast<uintptr_t>(p.y16) : reinterpret_cast<uintptr_t>(p.y);
+    const int wide = p.m % 4 == 0 && y % (epi == GEMM_BF16 ? 8 : 16) == 0;
+#define PLAMO_GEMM(EP) hipLaunchKernelGGL((gemm_small_kernel<EP, BT, BM, WT, WM, NT, H, NS>), grid, block, 0, s, p, cols, rows, wide)
     if (epi == GEMM_F32) PLAMO_GEMM(GEMM_F32);
     else if (epi == GEMM_BF16) PLAMO_GEMM(GEMM_BF16);
-    else if (epi == GEMM_RAW) PLAMO_GEMM(GEMM_RAW);
-    else if constexpr (TW % 2 == 0) PLAMO_GEMM(GEMM_SWIGLU);  // gate and up blocks pair inside a wave
-    else throw Error(E_INVAL, "SwiGLU GEMM needs an even number of column blocks per wave");
+    else PLAMO_GEMM(GEMM_RAW);
 #undef PLAMO_GEMM
+}
+
+template <int BT, int BM, int WT, int WM, int NT, int H, int NS>
+void launch_swiglu_small(const GemmParams& p, hipStream_t s) {
+    const int cols = INTER / (BM / 2), rows = (p.tokens + BT - 1) / BT, per = (cols * rows + 7) / 8;
+    const int wide = reinterpret_cast<uintptr_t>(p.y16) % 8 == 0;
+    hipLaunchKernelGGL((gemm_small_kernel<GEMM_SWIGLU, BT, BM, WT, WM, NT, H, NS>), dim3(8 * per), dim3(NT), 0, s, p,
+                       cols, rows, wide);
+}
+
+// A tile of the GEMM kernels and the measured time of one round of it (us; every CU one tile).
+struct GemmTile {
+    int bt, bm;
+    float us;
+    bool k256;  // its stages are 256 deep
+};
+// The tile whose rounds over the CUs take least: rounds = tiles / CUs, rounded up, since the
+// kernels run one workgroup per CU.  A call of few tokens thus takes the largest tiles that
+// still fill the chip, or small ones down to 16 x 16: every CU reads (bt + bm) rows of k values
+// however the tile is cut, so the smallest that fits one round is also the shortest.
+template <size_t N>
+int gemm_tile(const GemmTile (&tiles)[N], int cols, int tokens, int k) {
+    constexpr int CUS = 256;
+    int best = -1;
+    float least = 0.f;
+    for (size_t i = 0; i < N; ++i) {
+        const GemmTile& t = tiles[i];
+        if (t.k256 && k % 256 != 0) continue;
+        const int64_t n = int64_t((cols + t.bm - 1) / t.bm) * ((tokens + t.bt - 1) / t.bt);
+        const float us = float((n + CUS - 1) / CUS) * t.us;
+        if (best < 0 || us < least) best = int(i), least = us;
+    }
+    return best;
 }
 
 template <int BT, int BW, int WT, int NT>
@@ -1110,35 +1344,61 @@ void launch_gemm_packed(GemmEpilogue epi, const GemmParams& p, hipStream_t s) {
 }  // namespace
 
 void launch_gemm(bool packed, GemmEpilogue epi, const GemmParams& p, hipStream_t s) {
-    if (p.k % BK != 0 || p.tokens < 1 || p.m < 1 || (epi == GEMM_SWIGLU && p.m != 2 * INTER))
+    if (p.k % 128 != 0 || p.tokens < 1 || p.m < 1 || (epi == GEMM_SWIGLU && p.m != 2 * INTER))
         throw Error(E_INVAL, "unsupported GEMM shape");
     // operand and output views take 32-bit byte offsets (rows of the last tile included)
     const uint64_t t_pad = uint64_t(p.tokens) + 256;
     if (t_pad * uint64_t(p.k) * 2 >= (1ull << 31) || uint64_t(p.m) * uint64_t(p.k) * 2 >= (1ull << 31) ||
         t_pad * uint64_t(p.m) * 4 >= (1ull << 31))
         throw Error(E_INVAL, "GEMM operands exceed 2 GiB");
-    // Tile choice (measured on the prefill shapes, 2048 tokens): 256 x 128 tiles for the wide
-    // projections (gate_up, qkv), smaller ones for the 1536-row ones (o, down), where larger
-    // tiles leave CUs idle; plain weights go straight to LDS, .p12 weights are expanded in
-    // registers on the way.
-    const bool wide = p.tokens > 128 && (epi == GEMM_SWIGLU || p.m > 2048);
-    if (packed) {
-        if (wide) launch_gemm_packed<256, 128, 4, 512>(epi, p, s);
+    if (packed) {  // .p12 weights expanded in registers on the way to LDS
+        if (p.tokens > 128 && (epi == GEMM_SWIGLU || p.m > 2048)) launch_gemm_packed<256, 128, 4, 512>(epi, p, s);
         else launch_gemm_packed<128, 128, 2, 256>(epi, p, s);
-    } else {
-        // gate_up: 256 x 128 tiles on eight waves, three 64-deep stages (48 KB each): twice the
-        // MFMAs per barrier of 32-deep stages (gate_up 100 -> 72-77 us); 2048 tokens make 768
-        // tiles, three per CU
-        // qkv (2304 rows): 128 x 192 tiles on eight waves (192 tiles; 256 x 128 makes 144 and
-        // leaves 112 CUs idle): 22.3 -> 19.7-20.2 us at 2048 tokens
-        // 128 x 128 fallback (SwiGLU below 129 tokens): six 32-deep stages, five in flight
-        // 1536-row projections (o, down): 128 x 96 tiles with four waves, 64-deep stages, so
-        // 2048 tokens make exactly 256 tiles (128 x 128 left a quarter of the CUs idle)
-        if (wide && epi == GEMM_SWIGLU) launch_gemm_dma<256, 128, 4, 512, 64, 3>(epi, p, s);
-        else if (wide && p.m % 192 == 0) launch_gemm_dma<128, 192, 4, 512, 64, 3>(epi, p, s);
-        else if (wide) launch_gemm_dma<256, 128, 4, 512, 64, 3>(epi, p, s);
-        else if (epi != GEMM_SWIGLU && p.m % 96 == 0) launch_gemm_dma<128, 96, 4, 256, 64, 4>(epi, p, s);
-        else launch_gemm_dma<128, 128, 4, 512, 32, 6>(epi, p, s);
+        return;
+    }
+    // Tile choice: measured round times, cold weights.  gate_up (1536 deep), before (256 x 128
+    // and 128 x 128 tiles only) and now: 16 tokens 19.7 -> 9.1 us, 77 21.8 -> 12.1, 256 27.4 ->
+    // 20.4, 1024 53 -> 41, 1500 81 -> 69.
+    if (epi == GEMM_SWIGLU) {
+        static constexpr GemmTile tiles[] = {{16, 64, 9.1f, false},    {32, 64, 9.8f, false},   {64, 64, 11.5f, false},
+                                             {64, 96, 13.5f, false},   {128, 128, 19.5f, false}, {192, 128, 23.4f, false},
+                                             {256, 128, 28.2f, false}, {256, 192, 43.5f, false}};
+        switch (gemm_tile(tiles, 2 * INTER, p.tokens, p.k)) {
+            case 0: return launch_swiglu_small<16, 64, 1, 2, 128, 2, 4>(p, s);
+            case 1: return launch_swiglu_small<32, 64, 2, 2, 256, 2, 3>(p, s);
+            case 2: return launch_swiglu_small<64, 64, 4, 2, 512, 2, 3>(p, s);
+            case 3: return launch_swiglu_small<64, 96, 4, 1, 256, 1, 4>(p, s);
+            case 4: return launch_swiglu_small<128, 128, 2, 4, 512, 1, 4>(p, s);
+            case 5: return launch_swiglu_small<192, 128, 2, 4, 512, 1, 4>(p, s);
+            case 6: return launch_gemm_dma<256, 128, 4, 512, 3>(epi, p, s);
+            default: return launch_swiglu_small<256, 192, 4, 2, 512, 1, 2>(p, s);
+        }
+    }
+    // The other projections; round times of down (6144 deep; the ratios hold at 1536 and 2048).
+    // Before (128 x 96 and 128 x 192 tiles only) and now: down 16 tokens 36.9 -> 9.8 us, 77 43.4
+    // -> 12.8, 300 38.9 -> 18.7, 1024 46 -> 35, 1500 48 -> 41; o 16 tokens 14.5 -> 5.0, 300 15.2
+    // -> 7.9, 1024 17.1 -> 13.4; qkv 16 tokens 11.9 -> 4.6, 300 18.6 -> 8.1, 1024 19.7 -> 16.2.
+    static constexpr GemmTile tiles[] = {{16, 16, 9.7f, true},     {16, 16, 10.2f, false},  {32, 16, 10.8f, true},
+                                         {16, 32, 12.2f, false},   {32, 32, 14.0f, false},  {64, 32, 18.0f, false},
+                                         {64, 48, 23.5f, false},   {64, 64, 25.0f, false},  {96, 64, 28.5f, false},
+                                         {128, 64, 37.0f, false},  {64, 96, 35.0f, false},  {96, 96, 41.0f, false},
+                                         {128, 96, 49.0f, false},  {128, 128, 56.0f, false}, {128, 192, 74.0f, false}};
+    switch (gemm_tile(tiles, p.m, p.tokens, p.k)) {
+        case 0: return launch_gemm_small<16, 16, 1, 1, 256, 4, 6>(epi, p, s);
+        case 1: return launch_gemm_small<16, 16, 1, 1, 256, 2, 8>(epi, p, s);
+        case 2: return launch_gemm_small<32, 16, 2, 1, 256, 4, 4>(epi, p, s);
+        case 3: return launch_gemm_small<16, 32, 1, 2, 256, 2, 6>(epi, p, s);
+        case 4: return launch_gemm_small<32, 32, 2, 2, 256, 2, 4>(epi, p, s);
+        case 5: return launch_gemm_small<64, 32, 4, 1, 256, 2, 4>(epi, p, s);
+        case 6: return launch_gemm_small<64, 48, 4, 1, 256, 2, 3>(epi, p, s);
+        case 7: return launch_gemm_small<64, 64, 4, 2, 512, 2, 3>(epi, p, s);
+        case 8: return launch_gemm_small<96, 64, 2, 2, 256, 1, 4>(epi, p, s);
+        case 9: return launch_gemm_small<128, 64, 4, 2, 512, 1, 4>(epi, p, s);
+        case 10: return launch_gemm_small<64, 96, 4, 2, 512, 2, 3>(epi, p, s);
+        case 11: return launch_gemm_small<96, 96, 2, 2, 256, 1, 4>(epi, p, s);
+        case 12: return launch_gemm_dma<128, 96, 4, 256, 4>(epi, p, s);
+        case 13: return launch_gemm_small<128, 128, 2, 4, 512, 1, 4>(epi, p, s);
+        default: return launch_gemm_dma<128, 192, 4, 512, 3>(epi, p, s);
     }
 }
 
