@@ -406,10 +406,11 @@ __device__ __forceinline__ u32x4_t view_words(const void* base, uint32_t bytes) 
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
     return uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p));
 }
-__device__ __forceinline__ void load_to_lds_untracked(const u32x4_t view, uint32_t lds, uint32_t off) {
-    __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+__device__ __forceinline__ void load_to_lds_untracked(const u32x4_t view, uint32_t lds, uint32_t off, uint32_t scalar_off = 0) {
+    __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                      :
-                     : "s"(__builtin_amdgcn_readfirstlane(int(lds))), "v"(off), "s"(view)
+                     : "s"(__builtin_amdgcn_readfirstlane(int(lds))), "v"(off), "s"(view),
+                       "s"(__builtin_amdgcn_readfirstlane(int(scalar_off)))
                      : "m0", "memory");
 }
 
@@ -761,11 +762,6 @@ __global__ __launch_bounds__(256) void qk_prep_kernel(const QkPrepParams p) {
 constexpr int FT = 8;                 // tokens per query block (workgroup)
 constexpr int FK = 64;                // keys per tile
 static_assert(FT == 8 && FK == 64, "flash_block_tiles (prefill.h) assumes these sizes");
-// Direct path row strides (BF16 elements): key rows of 272 bytes (17 16-byte chunks, the
-// last one padding: consecutive rows start 4 banks apart), value rows of 320 bytes (20
-// chunks: 16 banks apart)
-constexpr int DK_ROW = 136, DV_ROW = 160;
-constexpr int DK_CHUNKS = DK_ROW / 8, DV_CHUNKS = DV_ROW / 8;
 constexpr int KST = HEAD_DIM + 8;     // K tile row stride (BF16), 16-byte aligned rows
 constexpr int VST = FK + 4;           // V^T tile row stride (BF16): 34 dwords, so 16 lanes reading
                                       // 8 bytes from 16 consecutive rows hit 32 distinct banks
@@ -856,15 +852,16 @@ __device__ __forceinline__ void flash_store(const KvSource& src, const KvStage& 
     }
 }
 
-// Two FP32 values as BF16 pairs hi + lo (RNE, v_cvt_pk_bf16_f32): hi + lo carries ~16
-// significant bits of each value.
+// Two FP32 values in [0, 1] as BF16 pairs hi + lo (RNE, v_cvt_pk_bf16_f32): hi + lo carries ~16
+// significant bits of each value.  The differences value - hi are exact, so one v_dot2_f32_bf16
+// each (hi times -1 and 0 onto the value) gives the same bits as unpacking hi and subtracting.
+// (The factors stay in registers: as literals the compiler encodes one as the inline constant
+// -1.0, which this instruction does not read as the pair (0, -1).)
 __device__ __forceinline__ void split_bf16(float a, float b, uint32_t& hw, uint32_t& lw) {
-    const floatx2 v = {a, b};
-    const bf16x2 h = __builtin_convertvector(v, bf16x2);
-    __builtin_memcpy(&hw, &h, 4);
-    const floatx2 back = {__uint_as_float(hw << 16), __uint_as_float(hw & 0xffff0000u)};
-    const bf16x2 l = __builtin_convertvector(v - back, bf16x2);
-    __builtin_memcpy(&lw, &l, 4);
+    uint32_t first = 0x0000bf80u, second = 0xbf800000u;
+    __asm__("" : "+s"(first), "+s"(second));
+    hw = pack_bf16(a, b);
+    lw = pack_bf16(dot2bf(hw, first, a), dot2bf(hw, second, b));
 }
 
 // Part `part` of query block qb.  QSA: global layers with a selection bitmap (a separate
@@ -872,14 +869,12 @@ __device__ __forceinline__ void split_bf16(float a, float b, uint32_t& hw, uint3
 template <bool QSA, bool DIRECT>
 __device__ __forceinline__ void flash_prefill(const FlashParams& p, const int qb, const int part) {
 #pragma clang fp contract(off)  // fixed rounding sequence, reproduced by the CPU oracle
-    // four distinct arrays (the compiler then tells the buffers apart and waits for the loads
-    // into one of them only before reading that one): K and V^T tiles of the staged path, or K
-    // and V tiles of the direct path, double-buffered
-    static_assert(FK * KST == FK * DK_ROW && HEAD_DIM * VST <= FK * DV_ROW, "tile buffers");
-    __shared__ __align__(1024) uint16_t L0[FK * DK_ROW];
-    __shared__ __align__(1024) uint16_t L1[FK * DK_ROW];
-    __shared__ __align__(1024) uint16_t L2[FK * DV_ROW];
-    __shared__ __align__(1024) uint16_t L3[FK * DV_ROW];
+    // two key and two value tiles: 16 KB each on the direct path; K rows and V^T, padded, on the
+    // staged one
+    constexpr int KT = FK * KST, VT = HEAD_DIM * VST;
+    __shared__ __align__(1024) uint8_t L[DIRECT ? 4 * FK * HEAD_DIM * 2 : 2 * (KT + VT) * 2];
+    uint16_t* const L0 = reinterpret_cast<uint16_t*>(L);
+    uint16_t *const L1 = L0 + KT, *const L2 = L1 + KT, *const L3 = L2 + VT;
     __shared__ int s_last;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, half = lane >> 5;
@@ -1051,75 +1046,56 @@ __device__ __forceinline__ void flash_prefill(const FlashParams& p, const int qb
         }
     } else {
         // (DIRECT: the launch holds only blocks whose keys need no rotation)
-        // Keys (already rotated) and values loaded straight into LDS (buffer loads with the
-        // LDS destination, no staging registers), in padded rows: key row R at R * 272 bytes
-        // (the S^T operand reads of 16 consecutive rows hit every bank), value row R at
-        // R * 320 bytes (the transposing V^T operand reads, ds_read_b64_tr_b16, of four rows x
-        // 64 bytes per half wave hit every bank).  Every operand read is one base address plus
-        // an immediate offset.  Tile j's keys and values go to buffer (j - j0) % 2 (L0/L1
-        // keys, L2/L3 values) and are requested at the start of tile j - 1.  Same arithmetic
-        // as the staged path.
-        // A tile is loaded as 16-byte chunks: chunk L of the tile (row L / chunks per row,
-        // piece L % chunks per row, pieces past 15 being padding) is lane L % 64 of load L / 64;
-        // wave w issues loads w, w + 4, ...  Its lanes' offsets within the tile are fixed: a
-        // tile whose 64 keys are consecutive ring slots without a wrap adds the first slot as
-        // a scalar offset; the last tile of a block (keys past khi load key khi) and tiles
-        // across the ring's end take per-lane slots.
-        constexpr int KLOADS = FK * DK_CHUNKS / 64, VLOADS = FK * DV_CHUNKS / 64;  // 17, 20
-        constexpr int KPER = (KLOADS + 3) / 4, VPER = VLOADS / 4;                 // 5, 5
-        static_assert(VLOADS % 4 == 0 && FK * DK_CHUNKS % 64 == 0, "tile loads");
-        const uint32_t krows = cached ? p.rot_rows : p.capacity;
-        const __amdgpu_buffer_rsrc_t kview = buffer_view(src.keys, krows * uint32_t(HEAD_DIM * 2));
-        const __amdgpu_buffer_rsrc_t vview = buffer_view(p.values, p.capacity * uint32_t(HEAD_DIM * 2));
-        // per load t of this wave: row (bits 0..7) and piece (bits 8..15) of this lane's chunk
-        uint32_t kpiece[KPER], vpiece[VPER];
+        // Keys (already rotated) and values loaded straight into LDS, two 16 KB tiles of each
+        // (tile j in buffer (j - j0) % 2).  Rows are 256 bytes, swizzled so that both operand
+        // reads hit every bank: 16-byte chunk c of key row R in slot c ^ (R % 16), 64-byte
+        // chunk d of value row R in slot d ^ (R % 4).  Tile j runs S^T of tile j + 1 beside the
+        // scaling and maximum of its own scores, then each quarter's exponentials beside the
+        // P.V products of the quarter before, in an order fixed by scheduling fences: a wave
+        // issues in order, and only so do the matrix cores work during its softmax.  Same
+        // arithmetic as the staged path.
+        const u32x4_t kview = view_words(src.keys, (cached ? p.rot_rows : p.capacity) * uint32_t(HEAD_DIM * 2));
+        const u32x4_t vview = view_words(p.values, p.capacity * uint32_t(HEAD_DIM * 2));
+        const int uw = __builtin_amdgcn_readfirstlane(wave);
+        const uint32_t lds = lds_address(L) + uint32_t(uw) * 4096u;
+        // load t of wave w: rows 16w + 4t .. + 3, lane l the slot l % 16 of row 16w + 4t + l / 16
+        const uint32_t lrow = uint32_t(16 * uw + (lane >> 4));
+        const uint32_t vsrc = lrow * 256u + (uint32_t((lane & 15) ^ ((lane >> 4) << 2)) << 4);
+        uint32_t ksrc[4];
 #pragma unroll
-        for (int t = 0; t < KPER; ++t) {
-            const int L = 64 * (wave + 4 * t) + lane;
-            kpiece[t] = uint32_t(L / DK_CHUNKS) | (uint32_t(L % DK_CHUNKS) << 8);
-        }
-#pragma unroll
-        for (int t = 0; t < VPER; ++t) {
-            const int L = 64 * (wave + 4 * t) + lane;
-            vpiece[t] = uint32_t(L / DV_CHUNKS) | (uint32_t(L % DV_CHUNKS) << 8);
-        }
-        auto tile_load = [&](const __amdgpu_buffer_rsrc_t view, uint16_t* dst, const uint32_t* piece, auto nloads,
-                             auto row_elems, int j, bool by_position) {
-            constexpr int N = decltype(nloads)::value, RE = decltype(row_elems)::value;
-            const uint32_t k0 = klo + uint32_t(j * FK);
-            const uint32_t slot0 = by_position ? k0 : k0 % p.capacity;
-            const bool plain = k0 + uint32_t(FK - 1) <= khi && (by_position || slot0 + uint32_t(FK - 1) < p.capacity);
-#pragma unroll
-            for (int t = 0; t < N; ++t) {
-                const int li = wave + 4 * t;
-                if (li * 64 >= FK * (RE / 8)) break;
-                const uint32_t row = piece[t] & 255u, pc = piece[t] >> 8;
-                uint32_t off;
-                if (plain) {
-                    off = row * uint32_t(HEAD_DIM * 2) + pc * 16u;
-                } else {
-                    const uint32_t kp = min(k0 + row, khi);
-                    uint32_t slot = by_position ? kp : slot0 + (kp - k0);
-                    slot = slot >= p.capacity && !by_position ? slot - p.capacity : slot;
-                    off = slot * uint32_t(HEAD_DIM * 2) + pc * 16u;
-                }
-                off = pc < 16u ? off : OOB_OFFSET;  // padding: nothing to load
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(view, (lds_ptr_t)(dst + li * 512), 16, off,
-                                                         plain ? int(slot0 * uint32_t(HEAD_DIM * 2)) : 0, 0, 0);
+        for (int t = 0; t < 4; ++t)
+            ksrc[t] = (lrow + uint32_t(4 * t)) * 256u + (uint32_t((lane & 15) ^ (lane >> 4) ^ (4 * t)) << 4);
+        uint32_t vfirst = (klo + uint32_t(j0 * FK)) % p.capacity;  // ring slot of the next value tile's first key
+        // Piece t of tile j's keys, and of the next value tile.  A tile whose 64 rows are
+        // consecutive adds its first row as a scalar; in a block's last tile rows past khi take key
+        // khi, and value rows wrap at the ring's end.  A tile past the part's end is its last
+        // again (nobody reads that copy).
+        auto request_k = [&](int j, auto piece) {
+            constexpr int t = decltype(piece)::value;
+            const uint32_t k0 = klo + uint32_t(min(j, j1 - 1) * FK);
+            const uint32_t dst = lds + uint32_t((j - j0) & 1) * 16384u + uint32_t(t) * 1024u;
+            if (k0 + uint32_t(FK - 1) <= khi) load_to_lds_untracked(kview, dst, ksrc[t], k0 * 256u);
+            else load_to_lds_untracked(kview, dst, min(lrow + uint32_t(4 * t), khi - k0) * 256u + (ksrc[t] & 255u), k0 * 256u);
+        };
+        auto request_v = [&](int j, auto piece) {
+            constexpr int t = decltype(piece)::value;
+            const uint32_t k0 = klo + uint32_t(min(j, j1 - 1) * FK);
+            const uint32_t dst = lds + 32768u + uint32_t((j - j0) & 1) * 16384u + uint32_t(t) * 1024u;
+            if (k0 + uint32_t(FK - 1) <= khi && vfirst + uint32_t(FK - 1) < p.capacity) {
+                load_to_lds_untracked(vview, dst, vsrc, vfirst * 256u + uint32_t(t) * 1024u);
+            } else {
+                const uint32_t slot = vfirst + min(lrow + uint32_t(4 * t), khi - k0);
+                load_to_lds_untracked(vview, dst, min(slot, slot - p.capacity) * 256u + (vsrc & 255u), 0u);
             }
         };
-        using KN = std::integral_constant<int, KPER>;
-        using VN = std::integral_constant<int, VPER>;
-        using KR = std::integral_constant<int, DK_ROW>;
-        using VR = std::integral_constant<int, DV_ROW>;
-        auto dma_k = [&](uint16_t* dst, int j) { tile_load(kview, dst, kpiece, KN{}, KR{}, j, cached || p.full); };
-        auto dma_v = [&](uint16_t* dst, int j) { tile_load(vview, dst, vpiece, VN{}, VR{}, j, false); };
+        auto advance_v = [&](int j) {  // to tile j
+            if (j < j1) vfirst += uint32_t(FK);
+            vfirst = vfirst >= p.capacity ? vfirst - p.capacity : vfirst;
+        };
         // S^T operand of row tile r, k-step s: key row 32r + col, dims 16s + 8 half .. + 8
-        auto kop_of = [&](const uint16_t* Kb) {
-            const uint16_t* base = Kb + col * DK_ROW + 8 * half;
-            return [=](int r, int s) {
-                return as_bf16x8(*reinterpret_cast<const uint4*>(base + 32 * r * DK_ROW + 16 * s));
-            };
+        const uint32_t kbase = uint32_t(col * 256 + ((half ^ (col & 15)) << 4));
+        auto kop = [&](int buf, int r, int s) {
+            return as_bf16x8(*reinterpret_cast<const uint4*>(L + buf * 16384 + r * 8192 + (kbase ^ uint32_t(s << 5))));
         };
         // V^T operand of d-tile dt, k-step s: source lane sl = lane % 16 of 16-lane group g =
         // lane / 16 addresses keys 16s + 4(g / 2) + sl / 4 (and + 8), dims 32dt + 16(g % 2) +
@@ -1129,102 +1105,217 @@ __device__ __forceinline__ void flash_prefill(const FlashParams& p, const int qb
         typedef short short4_t __attribute__((ext_vector_type(4)));
         typedef __attribute__((address_space(3))) short4_t* tr_ptr_t;
         const int sl = lane & 15, grp = lane >> 4;
-        const int vlane = (4 * (grp >> 1) + (sl >> 2)) * DV_ROW + 16 * (grp & 1) + 4 * (sl & 3);
-        auto vop_of = [&](const uint16_t* Vb) {
-            const uint16_t* base = Vb + vlane;
-            return [=](int dt, int s) {
-                const short4_t x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr_t)(base + 16 * s * DV_ROW + 32 * dt));
-                const short4_t x1 =
-                    __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr_t)(base + (16 * s + 8) * DV_ROW + 32 * dt));
-                bf16x8 a;
-                __builtin_memcpy(&a, &x0, 8);
-                __builtin_memcpy(reinterpret_cast<char*>(&a) + 8, &x1, 8);
-                return a;
+        const uint32_t vbase = uint32_t((4 * (grp >> 1) + (sl >> 2)) * 256 + ((sl >> 2) << 6) + 32 * (grp & 1) + 8 * (sl & 3));
+        auto vop = [&](int buf, int dt, int s) {
+            const uint8_t* at = L + 32768 + buf * 16384 + s * 4096 + (vbase ^ uint32_t(dt << 6));
+            const short4_t x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr_t)at);
+            const short4_t x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr_t)(at + 2048));
+            bf16x8 a;
+            __builtin_memcpy(&a, &x0, 8);
+            __builtin_memcpy(reinterpret_cast<char*>(&a) + 8, &x1, 8);
+            return a;
+        };
+        // Each wave waits for its own loads into LDS and its LDS reads, then the barrier: every
+        // tile requested so far is in, and the buffers of the tile before are free.
+        auto tiles_in = [&] {
+            __asm__ volatile("" ::: "memory");
+            wait_vmcnt_lds<0>();
+            __builtin_amdgcn_s_barrier();
+            __asm__ volatile("" ::: "memory");
+        };
+        // S^T product i (0..15) of the tile in buffer `buf`: k-step i / 2, row tile i % 2; its
+        // operand was read four products ago
+        bf16x8 kf[4];
+        auto st_first = [&](int buf) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) kf[i] = kop(buf, i & 1, i >> 1);
+        };
+        auto st = [&](int buf, auto n, floatx16 (&acc)[2]) {
+            constexpr int i = decltype(n)::value;
+            const floatx16 zero = {};
+            acc[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i & 3], qf[i >> 1], i < 2 ? zero : acc[i & 1], 0, 0, 0);
+            if constexpr (i + 4 < 16) kf[i & 3] = kop(buf, i & 1, (i + 4) >> 1);
+        };
+        auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
+
+        // Tile j (buffer B), whose scores are in sc; the scores of tile j + 1 go to sn (after the
+        // last tile: of stale keys, for nobody)
+        auto tile = [&](int j, auto par, floatx16 (&sc)[2], floatx16 (&sn)[2]) {
+            constexpr int B = decltype(par)::value;
+            tiles_in();
+            const uint32_t k0 = klo + uint32_t(j * FK);
+            const bool edge = QSA || !(k0 + uint32_t(FK - 1) <= plo && (p.full || k0 + uint32_t(WINDOW - 1) >= khi));
+            float mt = NEG_INF;
+            advance_v(j + 1);
+            st_first(B ^ 1);
+            // step n of sixteen: a product of S^T and, in the first eight, a request of a tile after
+            auto beside = [&](auto n) {
+                constexpr int i = decltype(n)::value;
+                if constexpr (i < 4) request_v(j + 1, std::integral_constant<int, i & 3>{});
+                else if constexpr (i < 8) request_k(j + 2, std::integral_constant<int, i & 3>{});
+                st(B ^ 1, n, sn);
             };
-        };
-        // tile j: its keys and values are in Kc / Vc; the next tile's go to Kn / Vn (free:
-        // read by tile j - 1 before this tile's barrier)
-        auto tile = [&](int j, const uint16_t* Kc, uint16_t* Kn, const uint16_t* Vc, uint16_t* Vn) {
-            // tile j is in (each wave waits for its own loads into LDS: the barrier's fence
-            // covers LDS operations, not loads into LDS, and every wave reads rows that other
-            // waves loaded); tile j - 1 is done with Kn and Vn
-            wait_vmcnt<0>();
-            __syncthreads();
-            if (j + 1 < j1) {
-                dma_k(Kn, j + 1);
-                dma_v(Vn, j + 1);
+            if (edge) {
+                // QSA (global layers: k0 is a multiple of 64): the tile's 16 blocks b0 .. b0 + 15
+                // are bits 0..15 of one bitmap word shifted by b0 % 32, read once per tile; blocks
+                // at or past qcomplete are not tested
+                uint32_t qbits = 0u;
+                const uint32_t b0 = k0 >> 2;
+                if (QSA && b0 < qcomplete) qbits = qmask[b0 >> 5] >> (b0 & 31) >> half;
+                // the lane's keys are k0 + 4 half + c for constants c
+                const int last = int(qpos - k0) - 4 * half, first = p.full ? -FK : last - (WINDOW - 1);
+                const int open = int(qcomplete - b0) - half;
+                static_for<0, 16>([&](auto n) {
+                    beside(n);
+#pragma unroll
+                    for (int e = 2 * decltype(n)::value; e < 2 * decltype(n)::value + 2; ++e) {
+                        const int r = e >> 4, q = e & 15, c = 32 * r + 8 * (q >> 2) + (q & 3), b = c >> 2;
+                        bool vis = c <= last && c >= first;
+                        if (QSA) vis = vis && (b >= open || ((qbits >> b) & 1u));
+                        const float x = vis ? sc[r][q] * SCALE_LOG2E : NEG_INF;
+                        sc[r][q] = x;
+                        mt = fmaxf(mt, x);
+                    }
+                    fence();
+                });
+            } else {
+                static_for<0, 16>([&](auto n) {
+                    constexpr int r = decltype(n)::value >> 3, q = 2 * decltype(n)::value & 15;
+                    beside(n);
+                    sc[r][q] = sc[r][q] * SCALE_LOG2E;
+                    sc[r][q + 1] = sc[r][q + 1] * SCALE_LOG2E;
+                    mt = fmaxf(fmaxf(mt, sc[r][q]), sc[r][q + 1]);
+                    fence();
+                });
             }
-            floatx16 sacc[2];
-            qk(sacc, kop_of(Kc));
-            softmax(j, sacc);
-            pv(sacc, vop_of(Vc));
+            mt = fmaxf(mt, xor_lane<32>(mt));
+            const float mn = fmaxf(m, mt);
+            const float ms = mn == NEG_INF ? 0.0f : mn;  // nothing visible yet: every p is 0
+            const float alpha = exp2_det(m - ms);
+            ls *= alpha;
+            m = mn;
+            // alpha is exactly 1 where the running maximum did not move: the wave skips the
+            // rescale when that holds in every lane (multiplying by 1 changes nothing)
+            if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+#pragma unroll
+                for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) oacc[dt][i] *= alpha;
+            }
+            // Quarter s: keys 16s + 4 half + {0..3} and 16s + 8 + 4 half + {0..3} as one k-step of
+            // P.V; product n of a quarter: d-tiles 0, 1 with hi then lo, then 2, 3
+            uint32_t hw[2][4], lw[2][4];
+            bf16x8 vf[2][2];
+            vf[0][0] = vop(B, 0, 0);
+            vf[0][1] = vop(B, 1, 0);
+            static_for<0, 20>([&](auto n) {
+                constexpr int s = decltype(n)::value >> 2, k = decltype(n)::value & 3;
+                if constexpr (s > 0) {
+                    constexpr int h = k >> 1, g = (s - 1) & 1;
+                    bf16x8 pw;
+                    if constexpr (k & 1) {
+                        pw = as_bf16x8(make_uint4(lw[g][0], lw[g][1], lw[g][2], lw[g][3]));
+                    } else {
+                        pw = as_bf16x8(make_uint4(hw[g][0], hw[g][1], hw[g][2], hw[g][3]));
+                        if constexpr (h == 0) {  // the operands of the next two d-tiles
+                            vf[1][0] = vop(B, 2, s - 1);
+                            vf[1][1] = vop(B, 3, s - 1);
+                        } else if constexpr (s < 4) {
+                            vf[0][0] = vop(B, 0, s);
+                            vf[0][1] = vop(B, 1, s);
+                        }
+                    }
+                    oacc[2 * h] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[h][0], pw, oacc[2 * h], 0, 0, 0);
+                    oacc[2 * h + 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[h][1], pw, oacc[2 * h + 1], 0, 0, 0);
+                }
+                if constexpr (s < 4) {
+                    constexpr int r = s >> 1, i = (s & 1) * 8 + 2 * k;
+                    const float e0 = exp2_det(sc[r][i] - ms), e1 = exp2_det(sc[r][i + 1] - ms);
+                    ls += e0;
+                    ls += e1;
+                    split_bf16(e0, e1, hw[s & 1][k], lw[s & 1][k]);
+                }
+                fence();
+            });
         };
-        dma_k(L0, j0);
-        dma_v(L2, j0);
+        floatx16 sa[2], sb[2];
+        static_for<0, 4>([&](auto t) { request_k(j0, t); });
+        static_for<0, 4>([&](auto t) { request_v(j0, t); });
+        tiles_in();
+        st_first(0);
+        static_for<0, 4>([&](auto t) { request_k(j0 + 1, t); });
+        static_for<0, 16>([&](auto n) { st(0, n, sa); });
         for (int j = j0; j < j1; j += 2) {
-            tile(j, L0, L1, L2, L3);
-            if (j + 1 < j1) tile(j + 1, L1, L0, L3, L2);
+            tile(j, std::integral_constant<int, 0>{}, sa, sb);
+            if (j + 1 < j1) tile(j + 1, std::integral_constant<int, 1>{}, sb, sa);
         }
+        wait_vmcnt<0>();  // no wave ends with a load into LDS in flight
     }
     // O = O^T / l; element i of d-tile dt is dim 32dt + 8(i/4) + 4*half + i%4
     float lt = ls + xor_lane<32>(ls);
     if (parts > 1) {
         // Partial (m, l, unnormalised O^T) of this part; the last part to finish merges all
         // parts of the block in part order: M = max m_q, w_q = 2^(m_q - M),
-        // O = sum O_q w_q / sum l_q w_q.
-        const int colg = wave * 32 + col;
+        // O = sum O_q w_q / sum l_q w_q.  A lane writes its sixteen 16-byte pieces where the same
+        // lane of the merging part reads them, whole lines per wave (in column order a part's
+        // 64 KB were 2,048 partial lines: 152 -> 136 us for 2048 queries from position 2048), and
+        // the merging part keeps its own in registers.
         const uint32_t nslots = uint32_t(flash_blocks(p.tokens)) * FLASH_PARTS;
         const __amdgpu_buffer_rsrc_t ov = buffer_view(p.part_o, nslots * (FT * HEADS) * HEAD_DIM * 4u);
         const __amdgpu_buffer_rsrc_t mv = buffer_view(p.part_ml, nslots * (FT * HEADS) * 8u);
-        auto o_off = [&](int q) { return uint32_t(((size_t(qb) * FLASH_PARTS + q) * (FT * HEADS) + colg) * HEAD_DIM * 4); };
-        auto ml_off = [&](int q) { return uint32_t(((size_t(qb) * FLASH_PARTS + q) * (FT * HEADS) + colg) * 8); };
+        auto o_off = [&](int q, int i) { return (uint32_t(qb * FLASH_PARTS + q) * 16u + uint32_t(i)) * 4096u + uint32_t(tid) * 16u; };
+        auto ml_off = [&](int q) { return (uint32_t(qb * FLASH_PARTS + q) * 128u + uint32_t(wave * 32 + col)) * 8u; };
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-                buffer_store16_sc1(ov, o_off(part) + (32 * dt + 8 * g + 4 * half) * 4,
-                                   make_uint4(__float_as_uint(oacc[dt][4 * g]), __float_as_uint(oacc[dt][4 * g + 1]),
-                                              __float_as_uint(oacc[dt][4 * g + 2]), __float_as_uint(oacc[dt][4 * g + 3])));
+        for (int i = 0; i < 16; ++i)
+            buffer_store16_sc1(ov, o_off(part, i),
+                               make_uint4(__float_as_uint(oacc[i >> 2][4 * (i & 3)]), __float_as_uint(oacc[i >> 2][4 * (i & 3) + 1]),
+                                          __float_as_uint(oacc[i >> 2][4 * (i & 3) + 2]), __float_as_uint(oacc[i >> 2][4 * (i & 3) + 3])));
         if (half == 0) buffer_store8_sc1(mv, ml_off(part), make_uint2(__float_as_uint(m), __float_as_uint(lt)));
         wait_stores();
         __syncthreads();
         if (tid == 0) s_last = atomicAdd(p.tickets + qb, 1u) == uint32_t(parts - 1);
         __syncthreads();
         if (!s_last) return;
-        float mq[FLASH_PARTS], lq[FLASH_PARTS];
-        float M = NEG_INF;
-#pragma unroll
-        for (int q = 0; q < FLASH_PARTS; ++q) {
-            if (q < parts) {
-                const uint2 v = buffer_load8_sc1(mv, ml_off(q));
-                mq[q] = __uint_as_float(v.x);
-                lq[q] = __uint_as_float(v.y);
-                M = fmaxf(M, mq[q]);
-            }
-        }
-        lt = 0.f;
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.f;
-#pragma unroll
-        for (int q = 0; q < FLASH_PARTS; ++q) {
-            if (q < parts) {
-                const float w = exp2_det(mq[q] - M);
-                lt += lq[q] * w;
-#pragma unroll
-                for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-                    for (int g = 0; g < 4; ++g) {
-                        const uint4 v = buffer_load16_sc1(ov, o_off(q) + (32 * dt + 8 * g + 4 * half) * 4);
-                        oacc[dt][4 * g] += __uint_as_float(v.x) * w;
-                        oacc[dt][4 * g + 1] += __uint_as_float(v.y) * w;
-                        oacc[dt][4 * g + 2] += __uint_as_float(v.z) * w;
-                        oacc[dt][4 * g + 3] += __uint_as_float(v.w) * w;
-                    }
-            }
-        }
         if (tid == 0) atomicExch(p.tickets + qb, 0u);  // ready for the next launch
+        // the other one or two parts, a before b, their outputs requested twelve pieces at a time
+        constexpr int BATCH = 12;
+        const int qa = part == 0 ? 1 : 0, qc = part == 2 ? 1 : 2;
+        const bool three = parts == 3;
+        const uint2 mla = buffer_load8_sc1(mv, ml_off(qa));
+        const uint2 mlb = three ? buffer_load8_sc1(mv, ml_off(qc)) : make_uint2(__float_as_uint(NEG_INF), 0u);
+        const float ma = __uint_as_float(mla.x), mb = __uint_as_float(mlb.x);
+        const float M = fmaxf(fmaxf(m, ma), mb);
+        const float w = exp2_det(m - M), wa = exp2_det(ma - M), wb = exp2_det(mb - M);
+        const float la = __uint_as_float(mla.y) * wa, lb = __uint_as_float(mlb.y) * wb, lown = lt * w;
+        // The sums in part order.  Without a third part its terms are +0 at the end, which change
+        // nothing (a sum that starts from +0 is never -0).
+        auto merge = [&](auto first, auto second, auto third) {
+            lt = ((0.f + first(lown, la, lb)) + second(lown, la, lb)) + third(lown, la, lb);
+            static_for<0, (16 + BATCH - 1) / BATCH>([&](auto batch) {
+                constexpr int i0 = decltype(batch)::value * BATCH, n = i0 + BATCH < 16 ? BATCH : 16 - i0;
+                uint4 va[n], vb[n];
+#pragma unroll
+                for (int i = 0; i < n; ++i) va[i] = buffer_load16_sc1(ov, o_off(qa, i0 + i));
+#pragma unroll
+                for (int i = 0; i < n; ++i) vb[i] = three ? buffer_load16_sc1(ov, o_off(qc, i0 + i)) : make_uint4(0, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < n; ++i) {
+                    const uint32_t xa[4] = {va[i].x, va[i].y, va[i].z, va[i].w}, xb[4] = {vb[i].x, vb[i].y, vb[i].z, vb[i].w};
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const int dt = (i0 + i) >> 2, e = 4 * ((i0 + i) & 3) + k;
+                        const float o = oacc[dt][e] * w, a = __uint_as_float(xa[k]) * wa, b = __uint_as_float(xb[k]) * wb;
+                        oacc[dt][e] = ((0.f + first(o, a, b)) + second(o, a, b)) + third(o, a, b);
+                    }
+                }
+            });
+        };
+        auto own = [](float o, float, float) { return o; };
+        auto pa = [](float, float a, float) { return a; };
+        auto pb = [](float, float, float b) { return b; };
+        if (part == 0) merge(own, pa, pb);
+        else if (part == 1) merge(pa, own, pb);
+        else merge(pa, pb, own);
     }
     if (!qvalid) return;
     uint16_t* orow = p.out + size_t(tq) * ATTN + head * HEAD_DIM;
