@@ -693,8 +693,8 @@ FlashWorkspace flash_workspace(int tokens) {
             (void)hipFree(w.tickets);
             w = FlashWorkspace{};
         }
-        PLAMO_HIP(hipMalloc(&w.o, plamo::flash_part_o_floats(tokens) * 4));
-        PLAMO_HIP(hipMalloc(&w.ml, plamo::flash_part_ml_floats(tokens) * 4));
+        PLAMO_HIP(hipMalloc(&w.o, plamo::flash_part_o_floats(plamo::flash_blocks(tokens)) * 4));
+        PLAMO_HIP(hipMalloc(&w.ml, plamo::flash_part_ml_floats(plamo::flash_blocks(tokens)) * 4));
         PLAMO_HIP(hipMalloc(&w.tickets, size_t(plamo::flash_blocks(tokens)) * 4));
         PLAMO_HIP(hipMemset(w.tickets, 0, size_t(plamo::flash_blocks(tokens)) * 4));
         w.tokens = tokens;
@@ -846,7 +846,7 @@ int plamo_kernel_attention_prefill(uint64_t q16, uint64_t keys, uint64_t values,
         f.out = reinterpret_cast<uint16_t*>(out16);
         f.capacity = uint32_t(capacity);
         f.p0 = uint32_t(p0);
-        f.tokens = tokens;
+        f.seg = plamo::one_segment(tokens);
         f.full = full ? 1 : 0;
         const FlashWorkspace ws = flash_workspace(tokens);
         f.part_o = ws.o;

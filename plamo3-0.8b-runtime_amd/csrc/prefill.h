@@ -33,6 +33,29 @@ struct RowsNormParams {
     int tokens;                // set by launch_rows_norm
 };
 
+// Rows of one prefill pass that belong to one KV lane: rows token0 .. token0 + tokens - 1 are its
+// tokens from position p0 on, and its query blocks (of 8 tokens) start at first_block.
+struct PrefillSegment {
+    int token0, tokens, first_block;
+    uint32_t lane;  // KV slice, counted from the one the pass's keys and values point to
+};
+constexpr int PREFILL_SEGMENTS = MAX_ROWS;
+struct PrefillSegments {
+    int n;
+    PrefillSegment s[PREFILL_SEGMENTS];
+    // the segment of row t, or of query block b
+    __host__ __device__ int of_token(int t) const {
+        int i = 0;
+        for (int k = 1; k < PREFILL_SEGMENTS; ++k) i = k < n && t >= s[k].token0 ? k : i;
+        return i;
+    }
+    __host__ __device__ int of_block(int b) const {
+        int i = 0;
+        for (int k = 1; k < PREFILL_SEGMENTS; ++k) i = k < n && b >= s[k].first_block ? k : i;
+        return i;
+    }
+};
+
 struct QkPrepParams {
     const uint16_t* qkv;       // [T][2304] BF16
     const uint16_t* q_norm;
@@ -44,6 +67,7 @@ struct QkPrepParams {
     uint32_t rot_rows;
     uint32_t capacity, p0;
     int tokens;
+    PrefillSegments seg;
     int full;
     const uint32_t* local_rope;   // [2064][64] BF16 (cos | sin << 16)
     const uint32_t* global_rope;  // [context][64]
@@ -54,6 +78,9 @@ struct QkPrepParams {
 constexpr int FLASH_PARTS = 3;
 constexpr int FLASH_PART_TILES = 11;         // 64-key tiles a part aims at
 __host__ __device__ inline int flash_blocks(int tokens) { return (tokens + 7) / 8; }
+inline int flash_blocks(const PrefillSegments& g) { return g.s[g.n - 1].first_block + flash_blocks(g.s[g.n - 1].tokens); }
+// One segment: `tokens` rows of the first KV slice.
+inline PrefillSegments one_segment(int tokens) { return PrefillSegments{1, {{0, tokens, 0, 0u}}}; }
 // workspace floats: per block and part, O^T [128 columns][128 dims] and (m, l) per column
 // Key tiles (64 keys) that query block qb of a call attends to, and the parts they are split
 // into (contiguous tile ranges, part q from q * tiles / parts).
@@ -70,13 +97,13 @@ __host__ __device__ inline int flash_block_parts(int tiles) {
 // The order in which workgroups take the (query block, part) items of a call: item w of the
 // launch is item[w] (qb << 2 | part).  n = 0: workgroup w takes part w / blocks of block
 // blocks - 1 - w % blocks (and returns if the block has fewer parts).
-constexpr int FLASH_SCHEDULE_MAX = 768;  // the items of a 2048-token call, at most
+constexpr int FLASH_SCHEDULE_MAX = 780;  // the items of a 2048-token pass of four segments, at most
 struct FlashSchedule {
     uint32_t n;
     uint16_t item[FLASH_SCHEDULE_MAX];
 };
-inline size_t flash_part_o_floats(int tokens) { return size_t(flash_blocks(tokens)) * FLASH_PARTS * 128 * 128; }
-inline size_t flash_part_ml_floats(int tokens) { return size_t(flash_blocks(tokens)) * FLASH_PARTS * 128 * 2; }
+inline size_t flash_part_o_floats(int blocks) { return size_t(blocks) * FLASH_PARTS * 128 * 128; }
+inline size_t flash_part_ml_floats(int blocks) { return size_t(blocks) * FLASH_PARTS * 128 * 2; }
 
 struct FlashParams {
     const uint16_t* q;         // [T][16][128] BF16, normalised and rotated
@@ -88,11 +115,12 @@ struct FlashParams {
     uint32_t rot_rows;
     uint16_t* out;             // [T][2048] BF16
     uint32_t capacity, p0;
-    int tokens;
+    PrefillSegments seg;
     int full;
-    float* part_o;             // flash_part_o_floats(tokens)
-    float* part_ml;            // flash_part_ml_floats(tokens)
-    uint32_t* tickets;         // flash_blocks(tokens), zero between launches
+    int blocks;                // query blocks of the pass (set by launch_flash_prefill)
+    float* part_o;             // flash_part_o_floats(blocks)
+    float* part_ml;            // flash_part_ml_floats(blocks)
+    uint32_t* tickets;         // one per block, zero between launches
     const uint32_t* qsa_mask;  // global layers with QSA: token t's selected blocks of four keys
                                // (bit b of word t * qsa_words + b / 32); null: every key
     uint32_t qsa_words;
@@ -102,5 +130,8 @@ void launch_gemm(bool packed, GemmEpilogue epi, const GemmParams& p, hipStream_t
 void launch_rows_norm(const RowsNormParams& p, int tokens, hipStream_t s);
 void launch_qk_prep(const QkPrepParams& p, hipStream_t s);
 void launch_flash_prefill(const FlashParams& p, hipStream_t s);
+// Every segment's last row of `a` and `b` ([rows][1536] BF16) to rows 0 .. n - 1 of `a_out` and `b_out`.
+void launch_gather_last(const uint16_t* a, const uint16_t* b, const PrefillSegments& seg, uint16_t* a_out, uint16_t* b_out,
+                        hipStream_t s);
 
 }  // namespace plamo

@@ -668,8 +668,10 @@ __global__ __launch_bounds__(256) void rows_norm_kernel(const RowsNormParams p) 
 __global__ __launch_bounds__(256) void qk_prep_kernel(const QkPrepParams p) {
     const int t = blockIdx.x, tid = threadIdx.x;
     const int hq = tid >> 4, sq = tid & 15;
-    const uint32_t pos = p.p0 + uint32_t(t);
-    const uint32_t chunk = p.p0 + (uint32_t(t) / CHUNK) * CHUNK;
+    const PrefillSegment sg = p.seg.s[p.seg.of_token(t)];
+    const uint32_t ts = uint32_t(t - sg.token0);  // the token within its segment
+    const uint32_t pos = p.p0 + ts;
+    const uint32_t chunk = p.p0 + (ts / CHUNK) * CHUNK;
     const uint32_t base = chunk > uint32_t(WINDOW - 1) ? chunk - uint32_t(WINDOW - 1) : 0u;
     const uint32_t qcoord = p.full ? pos : pos - base;
     const uint16_t* x = p.qkv + size_t(t) * QKV;
@@ -708,7 +710,7 @@ __global__ __launch_bounds__(256) void qk_prep_kernel(const QkPrepParams p) {
         *reinterpret_cast<uint2*>(qo + sq * 4) = make_uint2(pack_bf16(z[0], z[1]), pack_bf16(z[2], z[3]));
         *reinterpret_cast<uint2*>(qo + 64 + sq * 4) = make_uint2(pack_bf16(z[4], z[5]), pack_bf16(z[6], z[7]));
     }
-    const size_t slot = size_t(pos % p.capacity) * HEAD_DIM;
+    const size_t slot = (size_t(sg.lane) * p.capacity + pos % p.capacity) * HEAD_DIM;
     if (kthread) {
         float z[8];
         head_norm8(klo, khi, kgl, kgh, z);
@@ -721,7 +723,7 @@ __global__ __launch_bounds__(256) void qk_prep_kernel(const QkPrepParams p) {
             float zr[8] = {z[0], z[1], z[2], z[3], z[4], z[5], z[6], z[7]};
 #pragma unroll
             for (int j = 0; j < 4; j += 2) rope_pair_x2f(zr[j], zr[4 + j], c4[j], zr[j + 1], zr[4 + j + 1], c4[j + 1]);
-            uint16_t* kr = p.keys_rot + size_t(pos) * HEAD_DIM;
+            uint16_t* kr = p.keys_rot + (size_t(sg.lane) * p.rot_rows + pos) * HEAD_DIM;
             *reinterpret_cast<uint2*>(kr + tid * 4) = make_uint2(pack_bf16(zr[0], zr[1]), pack_bf16(zr[2], zr[3]));
             *reinterpret_cast<uint2*>(kr + 64 + tid * 4) = make_uint2(pack_bf16(zr[4], zr[5]), pack_bf16(zr[6], zr[7]));
         }
@@ -733,6 +735,14 @@ __global__ __launch_bounds__(256) void qk_prep_kernel(const QkPrepParams p) {
         const int d = tid - 64;
         p.values[slot + d] = x[ATTN + HEAD_DIM + d];
     }
+}
+
+__global__ __launch_bounds__(HIDDEN / 8) void gather_last_kernel(const uint16_t* a, const uint16_t* b,
+                                                                const PrefillSegments seg, uint16_t* a_out, uint16_t* b_out) {
+    const PrefillSegment sg = seg.s[blockIdx.x];
+    const size_t from = size_t(sg.token0 + sg.tokens - 1) * HIDDEN + threadIdx.x * 8, to = size_t(blockIdx.x) * HIDDEN + threadIdx.x * 8;
+    *reinterpret_cast<uint4*>(a_out + to) = *reinterpret_cast<const uint4*>(a + from);
+    *reinterpret_cast<uint4*>(b_out + to) = *reinterpret_cast<const uint4*>(b + from);
 }
 
 // --------------------------------------------------------------------- flash attention
@@ -867,8 +877,17 @@ __device__ __forceinline__ void split_bf16(float a, float b, uint32_t& hw, uint3
 // Part `part` of query block qb.  QSA: global layers with a selection bitmap (a separate
 // instance, so the dense kernel's edge tiles carry no bitmap test).
 template <bool QSA, bool DIRECT>
-__device__ __forceinline__ void flash_prefill(const FlashParams& p, const int qb, const int part) {
+__device__ __forceinline__ void flash_prefill(const FlashParams& pass, const int block, const int part) {
 #pragma clang fp contract(off)  // fixed rounding sequence, reproduced by the CPU oracle
+    // block `block` of the pass is block qb of its segment
+    const PrefillSegment sg = pass.seg.s[pass.seg.of_block(block)];
+    const int qb = block - sg.first_block, tokens = sg.tokens;
+    FlashParams p = pass;
+    p.q += size_t(sg.token0) * ATTN;
+    p.out += size_t(sg.token0) * ATTN;
+    p.keys += size_t(sg.lane) * p.capacity * HEAD_DIM;
+    p.values += size_t(sg.lane) * p.capacity * HEAD_DIM;
+    if (p.keys_rot) p.keys_rot += size_t(sg.lane) * p.rot_rows * HEAD_DIM;
     // two key and two value tiles: 16 KB each on the direct path; K rows and V^T, padded, on the
     // staged one
     constexpr int KT = FK * KST, VT = HEAD_DIM * VST;
@@ -879,10 +898,10 @@ __device__ __forceinline__ void flash_prefill(const FlashParams& p, const int qb
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, half = lane >> 5;
     const int t0 = qb * FT;
-    const int t1 = min(t0 + FT, p.tokens);
+    const int t1 = min(t0 + FT, tokens);
     const int tq = t0 + wave * 2 + (col >> 4);
     const int head = col & 15;
-    const bool qvalid = tq < p.tokens;
+    const bool qvalid = tq < tokens;
     const int tqc = qvalid ? tq : t1 - 1;
     const uint32_t qpos = p.p0 + uint32_t(tqc);
     const uint32_t chunk = p.p0 + (uint32_t(t0) / CHUNK) * CHUNK;
@@ -891,7 +910,7 @@ __device__ __forceinline__ void flash_prefill(const FlashParams& p, const int qb
     const uint32_t klo = p.full ? 0u : (plo > uint32_t(WINDOW - 1) ? plo - uint32_t(WINDOW - 1) : 0u);
     // The block's key tiles are split over up to FLASH_PARTS workgroups of about
     // FLASH_PART_TILES tiles each, so long (late) query blocks do not set the kernel's length.
-    const int ntiles = flash_block_tiles(p.tokens, p.p0, p.full, qb);
+    const int ntiles = flash_block_tiles(tokens, p.p0, p.full, qb);
     const int parts = flash_block_parts(ntiles);
     if (part >= parts) return;
     const int j0 = part * ntiles / parts, j1 = (part + 1) * ntiles / parts;
@@ -1260,11 +1279,11 @@ __device__ __forceinline__ void flash_prefill(const FlashParams& p, const int qb
         // lane of the merging part reads them, whole lines per wave (in column order a part's
         // 64 KB were 2,048 partial lines: 152 -> 136 us for 2048 queries from position 2048), and
         // the merging part keeps its own in registers.
-        const uint32_t nslots = uint32_t(flash_blocks(p.tokens)) * FLASH_PARTS;
+        const uint32_t nslots = uint32_t(p.blocks) * FLASH_PARTS;
         const __amdgpu_buffer_rsrc_t ov = buffer_view(p.part_o, nslots * (FT * HEADS) * HEAD_DIM * 4u);
         const __amdgpu_buffer_rsrc_t mv = buffer_view(p.part_ml, nslots * (FT * HEADS) * 8u);
-        auto o_off = [&](int q, int i) { return (uint32_t(qb * FLASH_PARTS + q) * 16u + uint32_t(i)) * 4096u + uint32_t(tid) * 16u; };
-        auto ml_off = [&](int q) { return (uint32_t(qb * FLASH_PARTS + q) * 128u + uint32_t(wave * 32 + col)) * 8u; };
+        auto o_off = [&](int q, int i) { return (uint32_t(block * FLASH_PARTS + q) * 16u + uint32_t(i)) * 4096u + uint32_t(tid) * 16u; };
+        auto ml_off = [&](int q) { return (uint32_t(block * FLASH_PARTS + q) * 128u + uint32_t(wave * 32 + col)) * 8u; };
 #pragma unroll
         for (int i = 0; i < 16; ++i)
             buffer_store16_sc1(ov, o_off(part, i),
@@ -1273,10 +1292,10 @@ __device__ __forceinline__ void flash_prefill(const FlashParams& p, const int qb
         if (half == 0) buffer_store8_sc1(mv, ml_off(part), make_uint2(__float_as_uint(m), __float_as_uint(lt)));
         wait_stores();
         __syncthreads();
-        if (tid == 0) s_last = atomicAdd(p.tickets + qb, 1u) == uint32_t(parts - 1);
+        if (tid == 0) s_last = atomicAdd(p.tickets + block, 1u) == uint32_t(parts - 1);
         __syncthreads();
         if (!s_last) return;
-        if (tid == 0) atomicExch(p.tickets + qb, 0u);  // ready for the next launch
+        if (tid == 0) atomicExch(p.tickets + block, 0u);  // ready for the next launch
         // the other one or two parts, a before b, their outputs requested twelve pieces at a time
         constexpr int BATCH = 12;
         const int qa = part == 0 ? 1 : 0, qc = part == 2 ? 1 : 2;
@@ -1339,7 +1358,7 @@ __device__ __forceinline__ void flash_prefill(const FlashParams& p, const int qb
 // XCD) and returns if the block has fewer parts.
 template <bool QSA, bool DIRECT>
 __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const FlashParams p) {
-    const int nqb = flash_blocks(p.tokens);
+    const int nqb = p.blocks;
     flash_prefill<QSA, DIRECT>(p, nqb - 1 - int(blockIdx.x) % nqb, int(blockIdx.x) / nqb);
 }
 
@@ -1499,6 +1518,11 @@ void launch_rows_norm(const RowsNormParams& p, int tokens, hipStream_t s) {
     hipLaunchKernelGGL(rows_norm_kernel, dim3((tokens + 3) / 4), dim3(256), 0, s, q);
 }
 
+void launch_gather_last(const uint16_t* a, const uint16_t* b, const PrefillSegments& seg, uint16_t* a_out, uint16_t* b_out,
+                        hipStream_t s) {
+    hipLaunchKernelGGL(gather_last_kernel, dim3(seg.n), dim3(HIDDEN / 8), 0, s, a, b, seg, a_out, b_out);
+}
+
 void launch_qk_prep(const QkPrepParams& p, hipStream_t s) {
     if (p.tokens < 1) return;
     hipLaunchKernelGGL(qk_prep_kernel, dim3(p.tokens), dim3(256), 0, s, p);
@@ -1518,26 +1542,29 @@ namespace {
 void flash_schedule(const FlashParams& p, FlashSchedule& sched) {
     // the last schedule of local and of global layers, per host thread
     thread_local struct {
-        int device = -1, cus = 0, tokens = -1;
+        int device = -1, cus = 0, tokens[PREFILL_SEGMENTS] = {-1};
         uint32_t p0 = 0;
         FlashSchedule sched{};
     } cache[2];
+    int lengths[PREFILL_SEGMENTS] = {};
+    for (int i = 0; i < p.seg.n; ++i) lengths[i] = p.seg.s[i].tokens;
     int device = 0;
     PLAMO_HIP(hipGetDevice(&device));
     auto& c = cache[p.full ? 1 : 0];
     if (c.device != device) {
         PLAMO_HIP(hipDeviceGetAttribute(&c.cus, hipDeviceAttributeMultiprocessorCount, device));
         c.device = device;
-        c.tokens = -1;
+        c.tokens[0] = -1;
     }
-    if (c.tokens != p.tokens || c.p0 != p.p0) {
+    if (!std::equal(lengths, lengths + PREFILL_SEGMENTS, c.tokens) || c.p0 != p.p0) {
         struct Item {
             int tiles, qb, part;
         };
         Item items[FLASH_SCHEDULE_MAX];
         int n = 0;
-        for (int qb = 0; qb < flash_blocks(p.tokens); ++qb) {
-            const int tiles = flash_block_tiles(p.tokens, p.p0, p.full, qb), parts = flash_block_parts(tiles);
+        for (int qb = 0; qb < p.blocks; ++qb) {
+            const PrefillSegment& sg = p.seg.s[p.seg.of_block(qb)];
+            const int tiles = flash_block_tiles(sg.tokens, p.p0, p.full, qb - sg.first_block), parts = flash_block_parts(tiles);
             for (int q = 0; q < parts; ++q) items[n++] = {(q + 1) * tiles / parts - q * tiles / parts, qb, q};
         }
         const int C = std::max(c.cus, 1);
@@ -1554,7 +1581,7 @@ void flash_schedule(const FlashParams& p, FlashSchedule& sched) {
             }
             c.sched.n = uint32_t(n);
         }
-        c.tokens = p.tokens;
+        std::copy(lengths, lengths + PREFILL_SEGMENTS, c.tokens);
         c.p0 = p.p0;
     }
     sched = c.sched;
@@ -1562,16 +1589,19 @@ void flash_schedule(const FlashParams& p, FlashSchedule& sched) {
 
 }  // namespace
 
-void launch_flash_prefill(const FlashParams& p, hipStream_t s) {
-    if (p.tokens < 1) return;
-    if (p.tokens > 65536 / FLASH_PARTS * 8) throw Error(E_INVAL, "flash prefill: too many tokens in one call");
+void launch_flash_prefill(const FlashParams& params, hipStream_t s) {
+    FlashParams p = params;
+    p.blocks = flash_blocks(p.seg);
+    if (p.blocks < 1) return;
+    if (p.blocks > 65536 / FLASH_PARTS) throw Error(E_INVAL, "flash prefill: too many tokens in one call");
     const bool qsa = p.full && p.qsa_mask;
     FlashSchedule sched;
     sched.n = 0;
-    if (flash_blocks(p.tokens) * FLASH_PARTS <= FLASH_SCHEDULE_MAX) flash_schedule(p, sched);
+    if (p.blocks * FLASH_PARTS <= FLASH_SCHEDULE_MAX) flash_schedule(p, sched);
     // keys straight into LDS when no block of the call rotates its keys: global layers, and
     // local layers whose keys all sit in the rotated-key cache (window base 0)
-    const uint32_t last = p.p0 + uint32_t(p.tokens) - 1;
+    uint32_t last = 0;
+    for (int i = 0; i < p.seg.n; ++i) last = std::max(last, p.p0 + uint32_t(p.seg.s[i].tokens) - 1);
     const bool direct = p.capacity >= uint32_t(FK) &&
                         (p.full || (p.keys_rot != nullptr && last < p.rot_rows && last < uint32_t(WINDOW)));
     const dim3 block(256);
@@ -1584,7 +1614,7 @@ void launch_flash_prefill(const FlashParams& p, hipStream_t s) {
         else PLAMO_FLASH(false, false);
 #undef PLAMO_FLASH
     } else {
-        const dim3 grid(uint32_t(flash_blocks(p.tokens) * FLASH_PARTS));
+        const dim3 grid(uint32_t(p.blocks * FLASH_PARTS));
 #define PLAMO_FLASH(Q, D) hipLaunchKernelGGL((flash_prefill_kernel<Q, D>), grid, block, 0, s, p)
         if (qsa) PLAMO_FLASH(true, true);
         else if (direct) PLAMO_FLASH(false, true);

@@ -108,7 +108,8 @@ class Engine {
     float *part_m, *part_l, *part_o;
     uint32_t* attn_tickets;
     uint32_t decode_parts_local, decode_parts_global;
-    // prefill scratch (chunk rows)
+    int pass_rows;           // rows of one prefill pass: a chunk, or several lanes' prompts
+    // prefill scratch (pass_rows rows)
     uint16_t *p_x, *p_qkv, *p_proj;  // BF16: every value is BF16-rounded
     uint16_t *p_xn, *p_att, *p_act, *p_q16;
     float *p_flash_o, *p_flash_ml;  // split flash prefill workspace
@@ -154,13 +155,16 @@ class Engine {
     void prepare_loop_graph();
     // prefill of `n` tokens of one lane at position p0 (n > 1); head on the last token.
     void prefill(const int32_t* tokens, int n, int p0, int lane, bool output);
+    // prefill of several lanes' whole prompts in one pass (seg: rows of `tokens`, KV lanes), at
+    // most pass_rows rows; segment q's logits, hidden row and prediction as row q of the state
+    void prefill_lanes(const int32_t* tokens, const PrefillSegments& seg);
     // after a prefill without output: the head of each of its first n rows, row i's logits,
     // final hidden row and prediction copied to slot i (the engine keeps row n - 1's)
     void prefill_heads(int n, uint16_t* slot_logits, float* slot_hidden, int32_t* slot_next);
     void zero_sampler();
 
   private:
-    void enqueue_prefill_chunk(int n, int p0, int lane, bool last_chunk, bool output);
+    void enqueue_prefill_pass(const PrefillSegments& seg, int n, int p0, int lane, bool output);
     void enqueue_head(const uint16_t* in, const uint16_t* resid_in, int in_rows);  // prefill rows
     void enqueue_head16(bool loop, int maxr);                                 // decode: BF16 stream
     void capture_loop(int steps, hipGraphExec_t* out);
