@@ -1468,11 +1468,12 @@ void launch_gemm(bool packed, GemmEpilogue epi, const GemmParams& p, hipStream_t
     }
     // Tile choice: measured round times, cold weights.  gate_up (1536 deep), before (256 x 128
     // and 128 x 128 tiles only) and now: 16 tokens 19.7 -> 9.1 us, 77 21.8 -> 12.1, 256 27.4 ->
-    // 20.4, 1024 53 -> 41, 1500 81 -> 69.
+    // 20.4, 400 25.4 -> 23.6, 1024 53 -> 41, 1500 81 -> 69.
     if (epi == GEMM_SWIGLU) {
         static constexpr GemmTile tiles[] = {{16, 64, 9.1f, false},    {32, 64, 9.8f, false},   {64, 64, 11.5f, false},
                                              {64, 96, 13.5f, false},   {128, 128, 19.5f, false}, {192, 128, 23.4f, false},
-                                             {256, 128, 28.2f, false}, {256, 192, 43.5f, false}};
+                                             {128, 192, 25.5f, false}, {256, 128, 28.2f, false},
+                                             {256, 192, 43.5f, false}};
         switch (gemm_tile(tiles, 2 * INTER, p.tokens, p.k)) {
             case 0: return launch_swiglu_small<16, 64, 1, 2, 128, 2, 4>(p, s);
             case 1: return launch_swiglu_small<32, 64, 2, 2, 256, 2, 3>(p, s);
@@ -1480,32 +1481,36 @@ void launch_gemm(bool packed, GemmEpilogue epi, const GemmParams& p, hipStream_t
             case 3: return launch_swiglu_small<64, 96, 4, 1, 256, 1, 4>(p, s);
             case 4: return launch_swiglu_small<128, 128, 2, 4, 512, 1, 4>(p, s);
             case 5: return launch_swiglu_small<192, 128, 2, 4, 512, 1, 4>(p, s);
-            case 6: return launch_gemm_dma<256, 128, 4, 512, 3>(epi, p, s);
+            case 6: return launch_swiglu_small<128, 192, 4, 2, 512, 1, 3>(p, s);
+            case 7: return launch_gemm_dma<256, 128, 4, 512, 3>(epi, p, s);
             default: return launch_swiglu_small<256, 192, 4, 2, 512, 1, 2>(p, s);
         }
     }
     // The other projections; round times of down (6144 deep; the ratios hold at 1536 and 2048).
-    // Before (128 x 96 and 128 x 192 tiles only) and now: down 16 tokens 36.9 -> 9.8 us, 77 43.4
-    // -> 12.8, 300 38.9 -> 18.7, 1024 46 -> 35, 1500 48 -> 41; o 16 tokens 14.5 -> 5.0, 300 15.2
-    // -> 7.9, 1024 17.1 -> 13.4; qkv 16 tokens 11.9 -> 4.6, 300 18.6 -> 8.1, 1024 19.7 -> 16.2.
-    static constexpr GemmTile tiles[] = {{16, 16, 9.7f, true},     {16, 16, 10.2f, false},  {32, 16, 10.8f, true},
+    // Before (128 x 96 and 128 x 192 tiles only) and now: down 16 tokens 36.9 -> 9.4 us, 77 43.4
+    // -> 12.3, 300 38.9 -> 18.7, 1024 46 -> 35, 1500 48 -> 40.5; o 16 tokens 14.5 -> 4.6, 300 15.2
+    // -> 7.9, 1024 17.1 -> 13.5; qkv 16 tokens 11.9 -> 4.2, 300 18.6 -> 8.1, 1024 19.7 -> 16.2.
+    // A small tile's time is the time to fill its stages, (bt + bm) rows through the CU's vector
+    // memory path: operands read a stage ahead, loads spread between the products, and
+    // activations loaded into registers instead of LDS all measured the same or slower.
+    static constexpr GemmTile tiles[] = {{16, 16, 9.4f, true},     {16, 16, 9.6f, false},   {32, 16, 10.5f, true},
                                          {16, 32, 12.2f, false},   {32, 32, 14.0f, false},  {64, 32, 18.0f, false},
-                                         {64, 48, 23.5f, false},   {64, 64, 25.0f, false},  {96, 64, 28.5f, false},
-                                         {128, 64, 37.0f, false},  {64, 96, 35.0f, false},  {96, 96, 41.0f, false},
+                                         {64, 48, 22.0f, false},   {64, 64, 25.0f, false},  {96, 64, 28.0f, false},
+                                         {128, 64, 37.0f, false},  {64, 96, 35.0f, false},  {96, 96, 40.0f, false},
                                          {128, 96, 49.0f, false},  {128, 128, 56.0f, false}, {128, 192, 74.0f, false}};
     switch (gemm_tile(tiles, p.m, p.tokens, p.k)) {
-        case 0: return launch_gemm_small<16, 16, 1, 1, 256, 4, 6>(epi, p, s);
+        case 0: return launch_gemm_small<16, 16, 1, 1, 256, 4, 4>(epi, p, s);
         case 1: return launch_gemm_small<16, 16, 1, 1, 256, 2, 8>(epi, p, s);
         case 2: return launch_gemm_small<32, 16, 2, 1, 256, 4, 4>(epi, p, s);
         case 3: return launch_gemm_small<16, 32, 1, 2, 256, 2, 6>(epi, p, s);
         case 4: return launch_gemm_small<32, 32, 2, 2, 256, 2, 4>(epi, p, s);
         case 5: return launch_gemm_small<64, 32, 4, 1, 256, 2, 4>(epi, p, s);
-        case 6: return launch_gemm_small<64, 48, 4, 1, 256, 2, 3>(epi, p, s);
+        case 6: return launch_gemm_small<64, 48, 4, 1, 256, 2, 4>(epi, p, s);
         case 7: return launch_gemm_small<64, 64, 4, 2, 512, 2, 3>(epi, p, s);
-        case 8: return launch_gemm_small<96, 64, 2, 2, 256, 1, 4>(epi, p, s);
+        case 8: return launch_gemm_small<96, 64, 2, 4, 512, 2, 3>(epi, p, s);
         case 9: return launch_gemm_small<128, 64, 4, 2, 512, 1, 4>(epi, p, s);
         case 10: return launch_gemm_small<64, 96, 4, 2, 512, 2, 3>(epi, p, s);
-        case 11: return launch_gemm_small<96, 96, 2, 2, 256, 1, 4>(epi, p, s);
+        case 11: return launch_gemm_small<96, 96, 2, 3, 384, 1, 4>(epi, p, s);
         case 12: return launch_gemm_dma<128, 96, 4, 256, 4>(epi, p, s);
         case 13: return launch_gemm_small<128, 128, 2, 4, 512, 1, 4>(epi, p, s);
         default: return launch_gemm_dma<128, 192, 4, 512, 3>(epi, p, s);

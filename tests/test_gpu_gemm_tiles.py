@@ -66,11 +66,11 @@ def test_gemm_tiles_bit_exact(m, n, tokens, skip):
     assert np.array_equal(_run(w, rows[of], 0, m, 4, skip), roundbf_np(want)[of])
 
 
-@pytest.mark.parametrize("tokens,skip", [(3, 0), (17, 0), (33, 1), (65, 0), (129, 0), (257, 0), (385, 0), (641, 2),
-                                         (1281, 0)])
+@pytest.mark.parametrize("tokens,skip", [(3, 0), (17, 0), (33, 1), (65, 0), (129, 0), (257, 0), (385, 0), (700, 2),
+                                         (1281, 0), (1537, 0)])
 def test_swiglu_tiles_bit_exact(tokens, skip):
-    """16 x 64, 32 x 64, 64 x 64, 64 x 96, 128 x 128, 192 x 128, 256 x 128, 256 x 192, 192 x 128 in
-    three rounds."""
+    """16 x 64, 32 x 64, 64 x 64, 64 x 96, 128 x 128, 192 x 128, 128 x 192, 256 x 192, 192 x 128 in
+    three rounds, 256 x 128."""
     print(f"  swiglu tokens={tokens}", flush=True)
     w, rows, of = _case(12288, 1536, tokens)
     want = xp.mfma_gemm(w, rows)
