@@ -353,11 +353,11 @@ int plamo_kernel_attention_decode(uint64_t qkv, uint64_t q_norm, uint64_t k_norm
 /* plamo_kernel_attention_decode without any device allocation.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same kernels and results;
- * the step state, tickets and partition buffers live in a static device array of
- * 4,260,352 bytes per GPU (held until the process ends), which limits every row to 8192
- * visible keys (global layers: pos < 8192): larger calls fail with PLAMO_EINVAL.  All calls
- * on one GPU share that array and every call rewrites the state and clears the tickets it
- * uses, so calls that overlap on one GPU (several streams or threads) race: serialise them.
+ * the tickets and partition buffers live in a static device array of 4,263,936 bytes
+ * per GPU (held until the process ends), which limits every row to 8192 visible keys (global
+ * layers: pos < 8192): larger calls fail with PLAMO_EINVAL.  All calls on one GPU share that
+ * array (its tickets are zero between calls), so calls that overlap on one GPU (several streams
+ * or threads) race: serialise them.
  * The caller passes every input and output, as for plamo_kernel_attention_decode. */
 int plamo_kernel_attention_decode_static(uint64_t qkv, uint64_t q_norm, uint64_t k_norm, uint64_t keys,
                                          uint64_t values, int32_t capacity, const int32_t* positions, int32_t rows,

@@ -1,4 +1,5 @@
 // extern "C" boundary (include/plamo_hip.h).  No C++ exception crosses it.
+#include <atomic>
 #include <chrono>
 #include <cstdio>
 #include <cstring>
@@ -702,9 +703,8 @@ FlashWorkspace flash_workspace(int tokens) {
     return w;
 }
 
-// Workspace of the kernel-level decode attention, per device, grown on demand: the step
-// state, the attention tickets [ROWS][4 head groups] and the partition statistics and
-// outputs [ROWS][parts][16] (x128 for the outputs), the layout the runtime's engine uses.
+// Workspace of the kernel-level decode attention (attn_workspace_bytes), per device, grown on
+// demand; the tickets are zero between calls.
 struct AttnWorkspace {
     void* base = nullptr;
     uint32_t parts = 0;
@@ -714,12 +714,13 @@ std::map<int, AttnWorkspace> g_attn_ws;
 
 
 // Carves a workspace at `base` (256-byte aligned) into the attention parameter pointers.
-void attn_workspace_bind(void* base, uint32_t parts, plamo::AttnParams& a, plamo::StepState*& st) {
-    uint8_t* b = static_cast<uint8_t*>(base);
+void attn_workspace_bind(void* base, uint32_t parts, plamo::AttnParams& a) {
+    // a set of tickets for each call: calls that overlap leave each other's alone
+    static std::atomic<uint32_t> calls{0};
+    uint32_t* tickets = static_cast<uint32_t*>(base);
     const size_t stats = size_t(plamo::ROWS) * parts * plamo::HEADS;
-    st = reinterpret_cast<plamo::StepState*>(b);
-    a.tickets = reinterpret_cast<uint32_t*>(b + 256);
-    a.part_m = reinterpret_cast<float*>(b + 512);
+    a.tickets = tickets + size_t(calls.fetch_add(1, std::memory_order_relaxed) % plamo::ATTN_TICKET_SETS) * plamo::ATTN_TICKETS;
+    a.part_m = reinterpret_cast<float*>(tickets + size_t(plamo::ATTN_TICKET_SETS) * plamo::ATTN_TICKETS);
     a.part_l = a.part_m + stats;
     a.part_o = a.part_l + stats;
 }
@@ -736,6 +737,7 @@ void* attn_workspace(uint32_t parts) {
             w = AttnWorkspace{};
         }
         PLAMO_HIP(hipMalloc(&w.base, plamo::attn_workspace_bytes(parts)));
+        PLAMO_HIP(hipMemset(w.base, 0, size_t(plamo::ATTN_TICKET_SETS) * plamo::ATTN_TICKETS * 4));
         w.parts = parts;
     }
     return w.base;
@@ -771,14 +773,15 @@ uint32_t attn_decode_params(uint64_t qkv, uint64_t q_norm, uint64_t k_norm, uint
     a.global_rope = reinterpret_cast<const uint32_t*>(global_rope);
     a.out16 = reinterpret_cast<uint16_t*>(out16);
     a.parts = uint32_t((most + plamo::KEYS_PER_PART - 1) / plamo::KEYS_PER_PART);
-    a.defer = full && a.parts > plamo::ATTN_MERGE_INLINE ? plamo::ATTN_MERGE_INLINE : 0;
+    // longer rows are merged by the merge kernel, on both kinds of layer as in the runtime
+    a.defer = a.parts > plamo::ATTN_MERGE_INLINE ? plamo::ATTN_MERGE_INLINE : 0;
+    a.window = full ? 0u : uint32_t(plamo::WINDOW);
+    a.state = nullptr;
+    for (int32_t q = 0; q < rows; ++q) a.arg_pos[q] = uint32_t(positions[q]);
     return a.parts;
 }
 
-void attn_decode_launch(plamo::AttnParams& a, plamo::StepState* st, const int32_t* positions, int32_t rows,
-                        bool full, hipStream_t s) {
-    a.state = st;
-    plamo::launch_attn_state(st, a.tickets, positions, rows, s);
+void attn_decode_launch(plamo::AttnParams& a, int32_t rows, bool full, hipStream_t s) {
     plamo::launch_attention(full, a, rows, s);
     if (a.defer) plamo::launch_attention_merge(a, rows, s);
 }
@@ -793,9 +796,8 @@ int plamo_kernel_attention_decode(uint64_t qkv, uint64_t q_norm, uint64_t k_norm
         plamo::AttnParams a{};
         const uint32_t parts = attn_decode_params(qkv, q_norm, k_norm, keys, values, capacity, positions, rows, full,
                                                   local_rope, global_rope, out16, a);
-        plamo::StepState* st = nullptr;
-        attn_workspace_bind(attn_workspace(parts), parts, a, st);
-        attn_decode_launch(a, st, positions, rows, full != 0, reinterpret_cast<hipStream_t>(stream));
+        attn_workspace_bind(attn_workspace(parts), parts, a);
+        attn_decode_launch(a, rows, full != 0, reinterpret_cast<hipStream_t>(stream));
         PLAMO_HIP(hipGetLastError());
     });
 }
@@ -812,9 +814,8 @@ int plamo_kernel_attention_decode_static(uint64_t qkv, uint64_t q_norm, uint64_t
             throw plamo::Error(plamo::E_INVAL, "attention exceeds the static scratch: at most " +
                                                    std::to_string(plamo::STATIC_ATTN_PARTS * plamo::KEYS_PER_PART) +
                                                    " visible keys per row");
-        plamo::StepState* st = nullptr;
-        attn_workspace_bind(plamo::static_attn_scratch(), parts, a, st);
-        attn_decode_launch(a, st, positions, rows, full != 0, reinterpret_cast<hipStream_t>(stream));
+        attn_workspace_bind(plamo::static_attn_scratch(), parts, a);
+        attn_decode_launch(a, rows, full != 0, reinterpret_cast<hipStream_t>(stream));
         PLAMO_HIP(hipGetLastError());
     });
 }

@@ -900,7 +900,9 @@ constexpr int KS = 68;               // padded LDS row of rotated keys: 64 BF16 
 // Workgroup (partition x, head group y, row z): keys x*64 .. x*64+63 of the row's visible
 // keys for heads 4y .. 4y+3.  All four head groups rotate the same keys; only group 0
 // writes the newest key and value to the cache.
-template <bool FULL>
+// ARGS: no step state, row q at position p.arg_pos[q] with KV slice q (kernel-level entry points,
+// whose state kernel in front cost as much as the attention: one local row at 344 keys 9.3 us).
+template <bool FULL, bool ARGS>
 __global__ __launch_bounds__(256) void attn_decode_kernel(const AttnParams p) {
 #pragma clang fp contract(off)  // fixed rounding sequence, reproduced by the CPU oracle
     PLAMO_TIMELINE_SCOPE(p.tag);
@@ -950,9 +952,9 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const AttnParams p) {
     // with coordinate r and the query with pos - first: a decode step is a 16-token chunk
     // of one token, whose RoPE base max(0, pos - 2047) is `first` (Runtime.swift:389,
     // Kernels.metal:251,283-284).
-    if (st->stopped || q >= int(st->rows)) return;
-    const uint32_t pos = st->pos[q];
-    const uint32_t lanei = st->kv_shared ? 0u : st->lane[q];
+    if (!ARGS && (st->stopped || q >= int(st->rows))) return;
+    const uint32_t pos = ARGS ? p.arg_pos[q] : st->pos[q];
+    const uint32_t lanei = ARGS ? uint32_t(q) : st->kv_shared ? 0u : st->lane[q];
     const uint32_t first = FULL ? 0u : (pos > uint32_t(WINDOW - 1) ? pos - uint32_t(WINDOW - 1) : 0u);
     const uint32_t qcoord = FULL ? pos : pos - first;
     const uint32_t count = pos + 1 - first;
@@ -1359,6 +1361,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const AttnParams p) {
 // few partitions in flight would take tens of microseconds at 500 partitions), then 32
 // threads sum in partition order.  Same arithmetic in the same order as the attention
 // kernel's own merge: M = max_p m_p, w_p = exp(m_p - M), den = sum l_p w_p, num = sum o_p w_p.
+template <bool ARGS>
 __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
 #pragma clang fp contract(off)  // fixed rounding sequence, reproduced by the CPU oracle
     PLAMO_TIMELINE_SCOPE(p.tag + 1);
@@ -1402,9 +1405,10 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
         if (k < early)
             ov[j] = buffer_load16_sc1(oview, uint32_t(((row0 + k) * HEADS + h) * HEAD_DIM + d0 + sub4) * 4u);
     }
-    if (st->stopped || q >= int(st->rows)) return;
+    if (!ARGS && (st->stopped || q >= int(st->rows))) return;
     // keys 0 .. pos on global layers, the last WINDOW of them on local layers
-    const uint32_t count = p.window && st->pos[q] + 1 > p.window ? p.window : st->pos[q] + 1;
+    const uint32_t seen = (ARGS ? p.arg_pos[q] : st->pos[q]) + 1;
+    const uint32_t count = p.window && seen > p.window ? p.window : seen;
     const uint32_t nparts = (count + KP - 1) / KP;
     if (nparts <= p.defer || nparts > MAXP || nparts > p.parts) return;  // merged in the attention kernel
 #pragma unroll
@@ -1720,7 +1724,6 @@ __global__ void unpack_kernel(const uint8_t* payload, const uint32_t* table, uin
 // copy per GPU, held until the process ends.  Host code uses the address hipGetSymbolAddress
 // returns for the current device (the array's name is not a device address on the host).
 static __device__ __align__(256) uint8_t scratch[attn_workspace_bytes(STATIC_ATTN_PARTS)];
-static_assert(sizeof(StepState) <= 256, "step state fits its workspace slot");
 
 }  // namespace
 
@@ -1741,26 +1744,6 @@ void* static_attn_scratch() {
 }
 
 namespace {
-
-struct AttnStateArgs {
-    int32_t pos[ROWS];
-    int32_t rows;
-};
-__global__ __launch_bounds__(64) void attn_state_kernel(StepState* st, uint32_t* tickets, AttnStateArgs a) {
-    const int tid = threadIdx.x;
-    uint32_t* w = reinterpret_cast<uint32_t*>(st);
-    for (int i = tid; i < STATE_WORDS; i += 64) w[i] = 0;
-    if (tid < ROWS * HEADS / HG) tickets[tid] = 0;
-    __syncthreads();
-    if (tid == 0) {
-        st->rows = uint32_t(a.rows);
-        st->penalty = 1.0f;
-        for (int q = 0; q < ROWS; ++q) {
-            st->lane[q] = uint32_t(q);
-            st->pos[q] = q < a.rows ? uint32_t(a.pos[q]) : 0u;
-        }
-    }
-}
 
 __global__ void fill_u32_kernel(uint32_t* p, uint32_t v, size_t n) {
     const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -1854,13 +1837,22 @@ void launch_gemv(int n, bool packed, int maxr, Prologue pro, Epilogue epi, const
 
 void launch_attention(bool full, const AttnParams& p, int rows, hipStream_t s) {
     const dim3 grid(32 * ((p.parts + 7) / 8), 1, rows), block(256);
-    if (full) hipLaunchKernelGGL(attn_decode_kernel<true>, grid, block, 0, s, p);
-    else hipLaunchKernelGGL(attn_decode_kernel<false>, grid, block, 0, s, p);
+#define PLAMO_ATTN(F, A) hipLaunchKernelGGL((attn_decode_kernel<F, A>), grid, block, 0, s, p)
+    if (p.state) {
+        if (full) PLAMO_ATTN(true, false);
+        else PLAMO_ATTN(false, false);
+    } else {
+        if (full) PLAMO_ATTN(true, true);
+        else PLAMO_ATTN(false, true);
+    }
+#undef PLAMO_ATTN
 }
 
 void launch_attention_merge(const AttnParams& p, int rows, hipStream_t s) {
     if (p.parts > uint32_t(MAX_CONTEXT / KEYS_PER_PART)) throw Error(E_INVAL, "attention merge: too many partitions");
-    hipLaunchKernelGGL(attn_merge_kernel, dim3(HEAD_DIM / 32, HEADS, rows), dim3(256), 0, s, p);
+    const dim3 grid(HEAD_DIM / 32, HEADS, rows);
+    if (p.state) hipLaunchKernelGGL(attn_merge_kernel<false>, grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL(attn_merge_kernel<true>, grid, dim3(256), 0, s, p);
 }
 
 void launch_head_merge(const DecodeBuffers& b, int blocks, bool begin_next, hipStream_t s) {
@@ -1893,13 +1885,6 @@ void launch_unpack(const uint8_t* payload, const uint32_t* table, uint16_t* out,
     if (count <= 0) return;
     if (count % 128) throw Error(E_INVAL, "unpack: count must be a whole number of 128-weight blocks");
     hipLaunchKernelGGL(unpack_kernel, dim3(unsigned((count / 8 + 255) / 256)), dim3(256), 0, s, payload, table, out, count);
-}
-
-void launch_attn_state(StepState* st, uint32_t* tickets, const int32_t* pos, int rows, hipStream_t s) {
-    AttnStateArgs a{};
-    for (int q = 0; q < ROWS; ++q) a.pos[q] = q < rows ? pos[q] : 0;
-    a.rows = rows;
-    hipLaunchKernelGGL(attn_state_kernel, dim3(1), dim3(64), 0, s, st, tickets, a);
 }
 
 void launch_fill_u32(uint32_t* p, uint32_t value, size_t count, hipStream_t s) {

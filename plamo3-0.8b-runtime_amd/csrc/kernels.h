@@ -45,7 +45,6 @@ struct StepState {
     // writes KV slice 0 at its own position; `lane` then only names its output slot.
     uint32_t kv_shared;
 };
-static_assert(sizeof(StepState) <= 256, "the kernel-level attention workspace keeps 256 B for the state");
 
 // Buffers the decode kernels share.
 struct DecodeBuffers {
@@ -102,7 +101,8 @@ struct GemvParams {
 };
 
 struct AttnParams {
-    const StepState* state;   // rows, positions and KV slices of the step
+    const StepState* state;   // rows, positions and KV slices of the step (null: arg_pos)
+    uint32_t arg_pos[ROWS];   // without a state: row q's position, its KV slice q
     uint32_t row0;            // the launch covers rows row0 .. row0 + gridDim.z - 1
     const float* qkv;         // [rows][2304] (BF16-valued FP32)
     const uint16_t* q_norm;   // [128]
@@ -202,23 +202,20 @@ void launch_unpack(const uint8_t* payload, const uint32_t* table, uint16_t* out,
 void launch_mtp_input(const float* hidden, const uint16_t* embed, int token, float* out, hipStream_t s);
 void launch_mtp_down(const float* up, const float* x, const uint16_t* w, float* out, hipStream_t s);
 void launch_fill_u32(uint32_t* p, uint32_t value, size_t count, hipStream_t s);
-// Device workspace of a kernel-level decode attention call, 256-byte aligned: the step state
-// (256 B), the attention tickets [ROWS][4 head groups] (256 B), then the partition
-// statistics m, l [ROWS][parts][16] and outputs [ROWS][parts][16][128] (FP32), the layout the
-// runtime's engine uses.
+// Device workspace of a kernel-level decode attention call, 256-byte aligned: ATTN_TICKET_SETS
+// sets of attention tickets [ROWS][4 head groups] (calls take them in turn; a set is zero
+// between its calls, since the last workgroup of a row and group clears its ticket), then the
+// partition statistics m, l [ROWS][parts][16] and outputs [ROWS][parts][16][128] (FP32), the
+// layout the runtime's engine uses.
+constexpr uint32_t ATTN_TICKET_SETS = 64, ATTN_TICKETS = ROWS * 4;
 constexpr size_t attn_workspace_bytes(uint32_t parts) {
-    return 512 + size_t(ROWS) * parts * 16 * (2 + 128) * 4;
+    return size_t(ATTN_TICKET_SETS) * ATTN_TICKETS * 4 + size_t(ROWS) * parts * 16 * (2 + 128) * 4;
 }
 // Partitions (64 keys each) the allocation-free entry point's static scratch holds: 8192 keys.
 constexpr uint32_t STATIC_ATTN_PARTS = 128;
 // Device address of this device's static scratch (attn_workspace_bytes(STATIC_ATTN_PARTS)
 // bytes), looked up once per device; every call on a device shares it.
 void* static_attn_scratch();
-
-// Step state of a kernel-level decode attention call: `rows` rows at `pos` (row q reads and
-// writes KV slice q), every other field zero; clears the rows' attention tickets.  Written by
-// a kernel from its arguments, so the call needs no host copy.
-void launch_attn_state(StepState* st, uint32_t* tickets, const int32_t* pos, int rows, hipStream_t s);
 
 // prefill.hip
 struct PrefillParams;
