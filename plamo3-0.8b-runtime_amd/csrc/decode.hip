@@ -1708,9 +1708,8 @@ __global__ __launch_bounds__(256) void mtp_down_kernel(const float* up, const fl
     if (lane == 0) out[r] = roundbf(x[r] + roundbf(t));
 }
 
-__global__ void unpack_kernel(const uint8_t* payload, const uint32_t* table, uint16_t* out, int64_t count) {
-    const int64_t i = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) * 8;
-    if (i >= count) return;
+// Weights i .. i + 7 of a .p12 tensor.
+__device__ __forceinline__ void unpack8(const uint8_t* payload, const uint32_t* table, uint16_t* out, int64_t i) {
     const uint32_t entry = table[i / 128];
     const uint8_t* blk = payload + (entry & ~63u);
     const uint32_t tag = entry & 63u, sub = uint32_t(i % 128) / 8;
@@ -1718,6 +1717,22 @@ __global__ void unpack_kernel(const uint8_t* payload, const uint32_t* table, uin
                              : p12_decode8(*reinterpret_cast<const uint2*>(blk + sub * 8),
                                            *reinterpret_cast<const uint32_t*>(blk + 128 + sub * 4), tag);
     *reinterpret_cast<uint4*>(out + i) = w;
+}
+
+__global__ void unpack_kernel(const uint8_t* payload, const uint32_t* table, uint16_t* out, int64_t count) {
+    const int64_t i = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) * 8;
+    if (i < count) unpack8(payload, table, out, i);
+}
+
+// Several tensors in one launch: tensor k takes the workgroups from first[k] on.  Bound by
+// memory (a layer's four projections: 54 MB in, 70 MB out) where a launch is long enough; one
+// tensor at a time, the small ones took 7 us for 12 MB.
+__global__ __launch_bounds__(256) void unpack_list_kernel(const UnpackList l) {
+    int k = 0;
+#pragma unroll
+    for (int j = 1; j < UNPACK_TENSORS; ++j) k = int(blockIdx.x) >= l.first[j] ? j : k;
+    const int64_t i = (int64_t(int(blockIdx.x) - l.first[k]) * 256 + threadIdx.x) * 8;
+    if (i < l.count[k]) unpack8(l.payload[k], l.table[k], l.out[k], i);
 }
 
 // Scratch of the allocation-free decode attention entry point: a file-scope device array, one
@@ -1885,6 +1900,16 @@ void launch_unpack(const uint8_t* payload, const uint32_t* table, uint16_t* out,
     if (count <= 0) return;
     if (count % 128) throw Error(E_INVAL, "unpack: count must be a whole number of 128-weight blocks");
     hipLaunchKernelGGL(unpack_kernel, dim3(unsigned((count / 8 + 255) / 256)), dim3(256), 0, s, payload, table, out, count);
+}
+
+void launch_unpack_list(UnpackList l, hipStream_t s) {
+    int blocks = 0;
+    for (int k = 0; k < UNPACK_TENSORS; ++k) {
+        if (l.count[k] % 128) throw Error(E_INVAL, "unpack: count must be a whole number of 128-weight blocks");
+        l.first[k] = blocks;
+        blocks += int((l.count[k] / 8 + 255) / 256);
+    }
+    hipLaunchKernelGGL(unpack_list_kernel, dim3(unsigned(blocks)), dim3(256), 0, s, l);
 }
 
 void launch_fill_u32(uint32_t* p, uint32_t value, size_t count, hipStream_t s) {

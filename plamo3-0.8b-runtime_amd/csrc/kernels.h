@@ -197,6 +197,16 @@ void launch_argmax(const void* x, uint32_t* out, int n, int rows, bool bf16, hip
 void launch_select(float* logits, int n, const int32_t* history, int hist, float penalty, int ngram, float frequency,
                    float presence, int32_t* out, hipStream_t s);
 void launch_unpack(const uint8_t* payload, const uint32_t* table, uint16_t* out, int64_t count, hipStream_t s);
+// A layer's four projections expanded in one launch (`first` is filled in by it).
+constexpr int UNPACK_TENSORS = 4;
+struct UnpackList {
+    const uint8_t* payload[UNPACK_TENSORS];
+    const uint32_t* table[UNPACK_TENSORS];
+    uint16_t* out[UNPACK_TENSORS];
+    int64_t count[UNPACK_TENSORS];
+    int first[UNPACK_TENSORS];
+};
+void launch_unpack_list(UnpackList l, hipStream_t s);
 // MTP adapter (Runtime.swift:485-520): input row [hidden | embed(token)], and the
 // activation + down projection + residual after the up projection (a 3072-wide GEMV).
 void launch_mtp_input(const float* hidden, const uint16_t* embed, int token, float* out, hipStream_t s);
