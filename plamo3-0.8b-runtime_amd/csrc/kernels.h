@@ -190,6 +190,10 @@ void launch_gemv(int n, bool packed, int maxr, Prologue pro, Epilogue epi, const
 // Rows p.row0 .. p.row0 + rows - 1 of the step (one launch per row for verification rows).
 void launch_attention(bool full, const AttnParams& p, int rows, hipStream_t s);
 void launch_attention_merge(const AttnParams& p, int rows, hipStream_t s);  // rows past the inline merge
+// The step state to the device, by value (the caller may change its copy at once), and back into
+// page-locked host memory (there once the stream has been waited for).
+void launch_state_put(StepState* state, const StepState& value, hipStream_t s);
+void launch_state_get(const StepState* state, StepState* host, hipStream_t s);
 void launch_step_begin(const DecodeBuffers& b, hipStream_t s);
 // begin_next: device loops run the next step's bookkeeping (step_begin) in the same kernel
 void launch_head_merge(const DecodeBuffers& b, int blocks, bool begin_next, hipStream_t s);

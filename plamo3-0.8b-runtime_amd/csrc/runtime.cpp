@@ -810,9 +810,11 @@ void RuntimeImpl::reset() {
 
 void RuntimeImpl::begin_timing() { PLAMO_HIP(hipEventRecord(eng->ev0, stream)); }
 
+// Ends the timed span, and the call: the state comes back behind it, in one wait for both.
 void RuntimeImpl::end_timing() {
     PLAMO_HIP(hipEventRecord(eng->ev1, stream));
-    PLAMO_HIP(hipEventSynchronize(eng->ev1));
+    launch_state_get(eng->state, eng->host_state, stream);
+    PLAMO_HIP(hipStreamSynchronize(stream));
     float ms = 0;
     PLAMO_HIP(hipEventElapsedTime(&ms, eng->ev0, eng->ev1));
     gpu_seconds += ms / 1000.0;
@@ -859,7 +861,7 @@ int RuntimeImpl::forward(const int32_t* tokens, int n, bool output) {
     hs.loop = 0;
     hs.stopped = 0;
     sync_sampler(e, 0);
-    PLAMO_HIP(hipMemcpyAsync(e.state, &hs, sizeof(StepState), hipMemcpyHostToDevice, stream));
+    launch_state_put(e.state, hs, stream);
     begin_timing();
     if (n == 1 && output) {
         e.run_step();
@@ -870,8 +872,6 @@ int RuntimeImpl::forward(const int32_t* tokens, int n, bool output) {
         e.prefill(tokens, n, int(position), 0, output);
     }
     end_timing();
-    PLAMO_HIP(hipMemcpyAsync(&hs, e.state, sizeof(StepState), hipMemcpyDeviceToHost, stream));
-    PLAMO_HIP(hipStreamSynchronize(stream));
     PLAMO_HIP(hipGetLastError());
     count_qsa(position, n);
     position += n;
@@ -896,12 +896,10 @@ int RuntimeImpl::prefill(const int32_t* tokens, int n) {
     hs.loop = 0;
     hs.stopped = 0;
     sync_sampler(e, 0);
-    PLAMO_HIP(hipMemcpyAsync(e.state, &hs, sizeof(StepState), hipMemcpyHostToDevice, stream));
+    launch_state_put(e.state, hs, stream);
     begin_timing();
     e.prefill(tokens, n, int(position), 0, true);
     end_timing();
-    PLAMO_HIP(hipMemcpyAsync(&hs, e.state, sizeof(StepState), hipMemcpyDeviceToHost, stream));
-    PLAMO_HIP(hipStreamSynchronize(stream));
     PLAMO_HIP(hipGetLastError());
     for (int s0 = 0; s0 < n; s0 += std::min(context, CHUNK))  // Runtime.fill's forwards (Runtime.swift:476)
         count_qsa(position + s0, std::min(std::min(context, CHUNK), n - s0));
@@ -941,7 +939,7 @@ int RuntimeImpl::forward_ex(const int32_t* tokens, int n, bool output, bool all,
         hs.kv_shared = 1;
         hs.loop = 0;
         hs.stopped = 0;
-        PLAMO_HIP(hipMemcpyAsync(e.state, &hs, sizeof(StepState), hipMemcpyHostToDevice, stream));
+        launch_state_put(e.state, hs, stream);
         e.run_verify();
         PLAMO_HIP(hipMemcpyAsync(aux->slot_logits, e.logits, size_t(VERIFY_ROWS) * VOCAB * 2, hipMemcpyDeviceToDevice,
                                  stream));
@@ -966,7 +964,7 @@ int RuntimeImpl::forward_ex(const int32_t* tokens, int n, bool output, bool all,
             hs.loop = 0;
             hs.stopped = 0;
             sync_sampler(e, 0);
-            PLAMO_HIP(hipMemcpyAsync(e.state, &hs, sizeof(StepState), hipMemcpyHostToDevice, stream));
+            launch_state_put(e.state, hs, stream);
             const bool head = output && (all || i == n - 1);
             if (head) e.run_step();
             else e.enqueue_step(false);
@@ -987,15 +985,16 @@ int RuntimeImpl::forward_ex(const int32_t* tokens, int n, bool output, bool all,
         hs.loop = 0;
         hs.stopped = 0;
         sync_sampler(e, 0);
-        PLAMO_HIP(hipMemcpyAsync(e.state, &hs, sizeof(StepState), hipMemcpyHostToDevice, stream));
+        launch_state_put(e.state, hs, stream);
         e.prefill(tokens, n, int(position), 0, false);
         if (output) e.prefill_heads(n, aux->slot_logits, aux->slot_hidden, aux->slot_next);
     }
     end_timing();
     int32_t next[VERIFY_ROWS] = {-1, -1};
-    if (rows > 1) PLAMO_HIP(hipMemcpyAsync(next, aux->slot_next, size_t(rows) * 4, hipMemcpyDeviceToHost, stream));
-    PLAMO_HIP(hipMemcpyAsync(&hs, e.state, sizeof(StepState), hipMemcpyDeviceToHost, stream));
-    PLAMO_HIP(hipStreamSynchronize(stream));
+    if (rows > 1) {
+        PLAMO_HIP(hipMemcpyAsync(next, aux->slot_next, size_t(rows) * 4, hipMemcpyDeviceToHost, stream));
+        PLAMO_HIP(hipStreamSynchronize(stream));
+    }
     PLAMO_HIP(hipGetLastError());
     hs.kv_shared = 0;  // later uploads run single rows again
     count_qsa(position, n);
@@ -1052,7 +1051,7 @@ int RuntimeImpl::draft(int first) {
     hs.loop = 0;
     hs.stopped = 0;
     hs.sampling = 0;
-    PLAMO_HIP(hipMemcpyAsync(e.state, &hs, sizeof(StepState), hipMemcpyHostToDevice, stream));
+    launch_state_put(e.state, hs, stream);
     GemvParams g{};
     g.state = e.state;
     g.rows = 1;
@@ -1066,8 +1065,6 @@ int RuntimeImpl::draft(int first) {
     launch_gemv(HIDDEN, m.packed, 1, PRO_PLAIN, EPI_LOGITS, g, head_blocks(1), stream);
     launch_head_merge(e.bufs, head_blocks(1), false, stream);
     end_timing();
-    PLAMO_HIP(hipMemcpyAsync(&hs, e.state, sizeof(StepState), hipMemcpyDeviceToHost, stream));
-    PLAMO_HIP(hipStreamSynchronize(stream));
     PLAMO_HIP(hipGetLastError());
     const int32_t d = int32_t(hs.next[0]);
     // the draft lands in the first prediction slot (Runtime.swift:503-507)
@@ -1150,13 +1147,13 @@ std::vector<int32_t> BatchImpl::prefill(const std::vector<std::vector<int32_t>>&
             if (group.size() > 1) tokens.insert(tokens.end(), p.begin(), p.end());
         }
         const auto& first = prompts[group[0]];
-        PLAMO_HIP(hipMemcpyAsync(e.state, &hs, sizeof(StepState), hipMemcpyHostToDevice, s));
+        launch_state_put(e.state, hs, s);
         PLAMO_HIP(hipEventRecord(e.ev0, s));
         if (group.size() > 1) e.prefill_lanes(tokens.data(), seg);
         else if (first.size() == 1) e.run_step();
         else e.prefill(first.data(), int(first.size()), 0, group[0], true);
         PLAMO_HIP(hipEventRecord(e.ev1, s));
-        PLAMO_HIP(hipMemcpyAsync(&hs, e.state, sizeof(StepState), hipMemcpyDeviceToHost, s));
+        launch_state_get(e.state, &hs, s);
         PLAMO_HIP(hipStreamSynchronize(s));
         PLAMO_HIP(hipGetLastError());
         float ms = 0;
@@ -1212,13 +1209,13 @@ std::vector<int32_t> BatchImpl::step(const std::vector<int32_t>& tokens) {
             active.push_back(int(i));
         }
     hs.rows = uint32_t(active.size());
-    PLAMO_HIP(hipMemcpyAsync(e.state, &hs, sizeof(StepState), hipMemcpyHostToDevice, s));
+    launch_state_put(e.state, hs, s);
     PLAMO_HIP(hipEventRecord(e.ev0, s));
     e.run_step();
     PLAMO_HIP(hipEventRecord(e.ev1, s));
     // Packed query rows are temporary; the head writes logits and hidden state at each row's
     // lane, so persistent outputs stay indexed by lane (Batch.swift:167-173).
-    PLAMO_HIP(hipMemcpyAsync(&hs, e.state, sizeof(StepState), hipMemcpyDeviceToHost, s));
+    launch_state_get(e.state, &hs, s);
     const hipError_t sync = hipStreamSynchronize(s);
     if (sync != hipSuccess) {
         ready = false;
@@ -1261,7 +1258,7 @@ BatchImpl::Decoded BatchImpl::decode(const std::vector<int32_t>& first, const st
         hs.llimit[i] = uint32_t(limits[i]);
         max_steps = std::max(max_steps, limits[i]);
     }
-    PLAMO_HIP(hipMemcpyAsync(e.state, &hs, sizeof(StepState), hipMemcpyHostToDevice, s));
+    launch_state_put(e.state, hs, s);
     PLAMO_HIP(hipEventRecord(e.ev0, s));
     // every step with running lanes emits a token on each of them, so the lane pass stops
     // the loop after at most max(limit) + 1 steps
@@ -1270,7 +1267,7 @@ BatchImpl::Decoded BatchImpl::decode(const std::vector<int32_t>& first, const st
     while (true) {
         e.run_steps(16);
         launched += 16;
-        PLAMO_HIP(hipMemcpyAsync(&hs, e.state, sizeof(StepState), hipMemcpyDeviceToHost, s));
+        launch_state_get(e.state, &hs, s);
         const hipError_t sync = hipStreamSynchronize(s);
         if (sync != hipSuccess) {
             ready = false;
@@ -1337,7 +1334,7 @@ std::vector<int32_t> RuntimeImpl::generate(const int32_t* prompt, int n, int max
     hs.reason = 0;
     hs.stopped = 0;
     sync_sampler(e, 0);
-    PLAMO_HIP(hipMemcpyAsync(e.state, &hs, sizeof(StepState), hipMemcpyHostToDevice, stream));
+    launch_state_put(e.state, hs, stream);
     begin_timing();
     e.begin_loop();
     int launched = 0;
@@ -1345,7 +1342,7 @@ std::vector<int32_t> RuntimeImpl::generate(const int32_t* prompt, int n, int max
         const int batch = std::min(16, max_tokens - launched);
         e.run_steps(batch);
         launched += batch;
-        PLAMO_HIP(hipMemcpyAsync(&hs, e.state, sizeof(StepState), hipMemcpyDeviceToHost, stream));
+        launch_state_get(e.state, &hs, stream);
         PLAMO_HIP(hipStreamSynchronize(stream));
         if (hs.stopped) break;
     }
@@ -1384,7 +1381,7 @@ double RuntimeImpl::bench_decode(int steps) {
     hs.reason = 0;
     hs.stopped = 0;
     sync_sampler(e, 0);
-    PLAMO_HIP(hipMemcpyAsync(e.state, &hs, sizeof(StepState), hipMemcpyHostToDevice, stream));
+    launch_state_put(e.state, hs, stream);
     e.prepare_loop_graph();  // captured outside the timed region (not run)
     e.begin_loop();
     e.run_steps(1);
@@ -1395,7 +1392,7 @@ double RuntimeImpl::bench_decode(int steps) {
     PLAMO_HIP(hipEventSynchronize(e.ev1));
     float ms = 0;
     PLAMO_HIP(hipEventElapsedTime(&ms, e.ev0, e.ev1));
-    PLAMO_HIP(hipMemcpyAsync(&hs, e.state, sizeof(StepState), hipMemcpyDeviceToHost, stream));
+    launch_state_get(e.state, &hs, stream);
     PLAMO_HIP(hipStreamSynchronize(stream));
     PLAMO_HIP(hipGetLastError());
     position = hs.pos[0];
