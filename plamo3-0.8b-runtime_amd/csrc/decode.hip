@@ -102,7 +102,12 @@ struct Staged {
     // as an input of an empty asm statement, so the compiler waits for its load), without
     // consuming them: requests issued after this call are not queued ahead of the inputs.
     __device__ __forceinline__ void wait_arrived() const {
-        if constexpr (PRO == PRO_PLAIN16) {
+        if constexpr (PRO == PRO_PLAIN) {
+#pragma unroll
+            for (int qi = 0; qi < RQ; ++qi)
+#pragma unroll
+                for (int k = 0; k < V; ++k) asm volatile("" ::"v"(v[qi][k].x), "v"(v[qi][k].y), "v"(v[qi][k].z), "v"(v[qi][k].w));
+        } else if constexpr (PRO == PRO_PLAIN16) {
 #pragma unroll
             for (int qi = 0; qi < RQ; ++qi)
 #pragma unroll
@@ -610,7 +615,10 @@ __global__ __launch_bounds__(64 * gemv_waves(N, MAXR, EPI)) void gemv_kernel(con
     WRaw<PACKED> wr[U][IT];
     if constexpr (PACKED) {
         // the payload as soon as the table arrived (the prologue loads issued after the table
-        // may still be in flight), then the next group's table
+        // may still be in flight), then the next group's table.  Four-row kernels hold it behind
+        // the inputs for the reason given below (four-row step 784 -> 737 us; the 6144-wide
+        // projection alone 9.6 -> 8.9 us).
+        if constexpr (MAXR > 1) S.wait_arrived();
         request_payload<U, IT>(p, tab, lane, wr);
         if (PIPE_TABLE && g + stride < gend) {
             int wrow[U];
