@@ -345,7 +345,9 @@ int plamo_kernel_attention_prefill(uint64_t q16, uint64_t keys, uint64_t values,
  * full != 0: keys 0..pos (global layer, pos < capacity, global_rope holds capacity rows of
  * [64] uint32 BF16 cos | sin << 16), else the 2048-key window ending at pos, keys rotated
  * with coordinate key_pos - max(0, pos - 2047) (local_rope: [2064][64]); out16: BF16
- * [rows][2048].  Uses a per-device workspace the library grows on demand. */
+ * [rows][2048].  Uses a per-device workspace the library grows on demand.  All calls on one GPU
+ * share it, so calls that overlap on one GPU (several streams, graphs or threads) race: serialise
+ * them.  The outputs of calls that did overlap are undefined; later calls are not affected. */
 int plamo_kernel_attention_decode(uint64_t qkv, uint64_t q_norm, uint64_t k_norm, uint64_t keys, uint64_t values,
                                   int32_t capacity, const int32_t* positions, int32_t rows, int32_t full,
                                   uint64_t local_rope, uint64_t global_rope, uint64_t out16, uint64_t stream);
@@ -353,11 +355,11 @@ int plamo_kernel_attention_decode(uint64_t qkv, uint64_t q_norm, uint64_t k_norm
 /* plamo_kernel_attention_decode without any device allocation.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same kernels and results;
- * the tickets and partition buffers live in a static device array of 4,263,936 bytes
+ * the tickets and partition buffers live in a static device array of 4,260,096 bytes
  * per GPU (held until the process ends), which limits every row to 8192 visible keys (global
  * layers: pos < 8192): larger calls fail with PLAMO_EINVAL.  All calls on one GPU share that
- * array (its tickets are zero between calls), so calls that overlap on one GPU (several streams
- * or threads) race: serialise them.
+ * array, so calls that overlap on one GPU race, as for plamo_kernel_attention_decode: serialise
+ * them.
  * The caller passes every input and output, as for plamo_kernel_attention_decode. */
 int plamo_kernel_attention_decode_static(uint64_t qkv, uint64_t q_norm, uint64_t k_norm, uint64_t keys,
                                          uint64_t values, int32_t capacity, const int32_t* positions, int32_t rows,

@@ -704,7 +704,7 @@ FlashWorkspace flash_workspace(int tokens) {
 }
 
 // Workspace of the kernel-level decode attention (attn_workspace_bytes), per device, grown on
-// demand; the tickets are zero between calls.
+// demand.
 struct AttnWorkspace {
     void* base = nullptr;
     uint32_t parts = 0;
@@ -712,17 +712,27 @@ struct AttnWorkspace {
 std::mutex g_attn_ws_mu;
 std::map<int, AttnWorkspace> g_attn_ws;
 
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (s) PLAMO_HIP(hipStreamIsCapturing(s, &status));  // the default stream cannot be captured
+    return status != hipStreamCaptureStatusNone;
+}
 
-// Carves a workspace at `base` (256-byte aligned) into the attention parameter pointers.
-void attn_workspace_bind(void* base, uint32_t parts, plamo::AttnParams& a) {
-    // a set of tickets for each call: calls that overlap leave each other's alone
-    static std::atomic<uint32_t> calls{0};
-    uint32_t* tickets = static_cast<uint32_t*>(base);
+// Carves a workspace at `base` (256-byte aligned) into the attention parameter pointers and takes
+// the call's tickets in it.
+void attn_workspace_bind(void* base, uint32_t parts, plamo::AttnParams& a, hipStream_t s) {
+    static std::atomic<uint64_t> calls{0};
+    uint64_t* tickets = static_cast<uint64_t*>(base);
     const size_t stats = size_t(plamo::ROWS) * parts * plamo::HEADS;
-    a.tickets = tickets + size_t(calls.fetch_add(1, std::memory_order_relaxed) % plamo::ATTN_TICKET_SETS) * plamo::ATTN_TICKETS;
-    a.part_m = reinterpret_cast<float*>(tickets + size_t(plamo::ATTN_TICKET_SETS) * plamo::ATTN_TICKETS);
+    a.call = (calls.fetch_add(1, std::memory_order_relaxed) + 1) << 8;
+    a.call_tickets = tickets;
+    a.part_m = reinterpret_cast<float*>(tickets + 2 * plamo::ATTN_TICKETS);
     a.part_l = a.part_m + stats;
     a.part_o = a.part_l + stats;
+    if (parts > 1 && capturing(s)) {
+        a.call_tickets += plamo::ATTN_TICKETS;
+        plamo::launch_fill_u32(reinterpret_cast<uint32_t*>(a.call_tickets), 0, size_t(plamo::ATTN_TICKETS) * 2, s);
+    }
 }
 
 void* attn_workspace(uint32_t parts) {
@@ -737,7 +747,7 @@ void* attn_workspace(uint32_t parts) {
             w = AttnWorkspace{};
         }
         PLAMO_HIP(hipMalloc(&w.base, plamo::attn_workspace_bytes(parts)));
-        PLAMO_HIP(hipMemset(w.base, 0, size_t(plamo::ATTN_TICKET_SETS) * plamo::ATTN_TICKETS * 4));
+        PLAMO_HIP(hipMemset(w.base, 0, size_t(2) * plamo::ATTN_TICKETS * 8));
         w.parts = parts;
     }
     return w.base;
@@ -796,7 +806,7 @@ int plamo_kernel_attention_decode(uint64_t qkv, uint64_t q_norm, uint64_t k_norm
         plamo::AttnParams a{};
         const uint32_t parts = attn_decode_params(qkv, q_norm, k_norm, keys, values, capacity, positions, rows, full,
                                                   local_rope, global_rope, out16, a);
-        attn_workspace_bind(attn_workspace(parts), parts, a);
+        attn_workspace_bind(attn_workspace(parts), parts, a, reinterpret_cast<hipStream_t>(stream));
         attn_decode_launch(a, rows, full != 0, reinterpret_cast<hipStream_t>(stream));
         PLAMO_HIP(hipGetLastError());
     });
@@ -814,7 +824,7 @@ int plamo_kernel_attention_decode_static(uint64_t qkv, uint64_t q_norm, uint64_t
             throw plamo::Error(plamo::E_INVAL, "attention exceeds the static scratch: at most " +
                                                    std::to_string(plamo::STATIC_ATTN_PARTS * plamo::KEYS_PER_PART) +
                                                    " visible keys per row");
-        attn_workspace_bind(plamo::static_attn_scratch(), parts, a);
+        attn_workspace_bind(plamo::static_attn_scratch(), parts, a, reinterpret_cast<hipStream_t>(stream));
         attn_decode_launch(a, rows, full != 0, reinterpret_cast<hipStream_t>(stream));
         PLAMO_HIP(hipGetLastError());
     });

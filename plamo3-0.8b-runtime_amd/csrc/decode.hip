@@ -1005,6 +1005,12 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const AttnParams p) {
     const __amdgpu_buffer_rsrc_t oview = buffer_view(p.part_o, pstats * HEAD_DIM * 4u);
     const uint32_t nparts = (count + KP - 1) / KP;
     if (part >= nparts) return;  // partitions past the visible keys take no ticket
+    using Ticket = std::conditional_t<ARGS, unsigned long long, uint32_t>;
+    Ticket* ticket;
+    if constexpr (ARGS) ticket = reinterpret_cast<Ticket*>(p.call_tickets);
+    else ticket = p.tickets;
+    ticket += q * (HEADS / HG) + hg;
+    const Ticket base = ARGS ? Ticket(p.call) : Ticket(0);
     const uint32_t newest = count - 1;
     const bool has_new = newest >= k0 && newest < k0 + KP;
 
@@ -1164,6 +1170,11 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const AttnParams p) {
             if (nparts > 1) {
                 buffer_store4_sc1(mview, uint32_t(pslot * HEADS + hg * HG + w) * 4u, __float_as_uint(m));
                 buffer_store4_sc1(lview, uint32_t(pslot * HEADS + hg * HG + w) * 4u, __float_as_uint(l));
+                // Without a state, a ticket that is taken below is first raised to this call's
+                // number (a zero, or what an earlier call left, falls to it): on its way during
+                // P.V, in before the wait for this wave's stores (14 calls of one local row at 344
+                // keys 102 us, as with tickets taken to be zero; raised at that wait 104).
+                if (ARGS && w == 0 && (p.defer == 0 || nparts <= p.defer)) atomicMax(ticket, base);
             }
         }
     }
@@ -1219,11 +1230,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const AttnParams p) {
     // wave's partition stores have completed before the ticket is taken
     wait_stores();
     __syncthreads();
-    uint32_t* ticket = p.tickets + q * (HEADS / HG) + hg;
-    if (tid == 0) {
-        const uint32_t prev = atomicAdd(ticket, 1u);
-        s_last = prev == nparts - 1;
-    }
+    if (tid == 0) s_last = atomicAdd(ticket, Ticket(1)) == base + nparts - 1;
     __syncthreads();
     if (!s_last) return;
     const size_t row0 = size_t(q) * p.parts;
@@ -1380,7 +1387,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const AttnParams p) {
         for (int i = 0; i < 2; ++i)
             p.out16[size_t(q) * ATTN + (hg * HG + hb + 2 * i) * HEAD_DIM + d] = uint16_t(bits(num[i] / den_s[hb + 2 * i]));
     }
-    if (tid == 0) atomicExch(ticket, 0u);  // ready for the next launch
+    if (tid == 0) atomicExch(ticket, Ticket(0));  // ready for the next launch
 }
 
 // Partition merge of rows with more than p.defer partitions (long contexts),

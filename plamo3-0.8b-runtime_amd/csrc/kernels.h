@@ -119,7 +119,12 @@ struct AttnParams {
     float* part_l;
     float* part_o;            // [ROWS][parts][16][128]
     uint32_t parts;           // grid.x
-    uint32_t* tickets;        // [rows][head groups], zero between launches
+    uint32_t* tickets;        // [rows][head groups], zero between launches (with a state)
+    // Without a state: the call's number, which grows from call to call, and its tickets, each the
+    // number of the call that holds it and that call's count: a count that another call left behind
+    // is never added to.
+    uint64_t call;            // number << 8
+    uint64_t* call_tickets;   // [rows][head groups]
     uint16_t* out16;          // BF16 [rows][2048]
     uint32_t defer;           // rows with more partitions than this (0: none) are merged by
                               // attn_merge_kernel instead of the attention kernel's last workgroup
@@ -216,14 +221,14 @@ void launch_unpack_list(UnpackList l, hipStream_t s);
 void launch_mtp_input(const float* hidden, const uint16_t* embed, int token, float* out, hipStream_t s);
 void launch_mtp_down(const float* up, const float* x, const uint16_t* w, float* out, hipStream_t s);
 void launch_fill_u32(uint32_t* p, uint32_t value, size_t count, hipStream_t s);
-// Device workspace of a kernel-level decode attention call, 256-byte aligned: ATTN_TICKET_SETS
-// sets of attention tickets [ROWS][4 head groups] (calls take them in turn; a set is zero
-// between its calls, since the last workgroup of a row and group clears its ticket), then the
-// partition statistics m, l [ROWS][parts][16] and outputs [ROWS][parts][16][128] (FP32), the
+// Device workspace of a kernel-level decode attention call, 256-byte aligned: two sets of
+// attention tickets [ROWS][4 head groups] (the first for calls that run at once, the second for
+// calls that a graph records, which clear it themselves: a replay's number is an old one), then
+// the partition statistics m, l [ROWS][parts][16] and outputs [ROWS][parts][16][128] (FP32), the
 // layout the runtime's engine uses.
-constexpr uint32_t ATTN_TICKET_SETS = 64, ATTN_TICKETS = ROWS * 4;
+constexpr uint32_t ATTN_TICKETS = ROWS * 4;
 constexpr size_t attn_workspace_bytes(uint32_t parts) {
-    return size_t(ATTN_TICKET_SETS) * ATTN_TICKETS * 4 + size_t(ROWS) * parts * 16 * (2 + 128) * 4;
+    return size_t(2) * ATTN_TICKETS * 8 + size_t(ROWS) * parts * 16 * (2 + 128) * 4;
 }
 // Partitions (64 keys each) the allocation-free entry point's static scratch holds: 8192 keys.
 constexpr uint32_t STATIC_ATTN_PARTS = 128;
