@@ -329,7 +329,9 @@ int plamo_kernel_gemm(uint64_t w, uint64_t table, uint64_t x, uint64_t y, int32_
  * [capacity][128] with position p in slot p % capacity (keys of global layers rotated at
  * their position, local keys unrotated); full != 0: causal over all keys, else the
  * 2048-key window with keys rotated at key_pos - base of each 16-token chunk
- * (local_rope: [2064][64] uint32 = BF16 cos | sin << 16).  out16: BF16 [tokens][2048]. */
+ * (local_rope: [2064][64] uint32 = BF16 cos | sin << 16).  out16: BF16 [tokens][2048].
+ * Queries with more than 11 tiles of 64 visible keys use a per-device workspace the library
+ * grows on demand: such calls have to be serialised, as for plamo_kernel_attention_decode. */
 int plamo_kernel_attention_prefill(uint64_t q16, uint64_t keys, uint64_t values, int32_t capacity, int32_t p0,
                                    int32_t tokens, int32_t full, uint64_t local_rope, uint64_t out16,
                                    uint64_t stream);

@@ -670,6 +670,24 @@ int plamo_kernel_gemm(uint64_t w, uint64_t table, uint64_t x, uint64_t y, int32_
 }  // extern "C" (the helper below is C++ only)
 
 namespace {
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (s) PLAMO_HIP(hipStreamIsCapturing(s, &status));  // the default stream cannot be captured
+    return status != hipStreamCaptureStatusNone;
+}
+
+// Tickets of a workspace that has just grown are cleared on the stream of the call that uses them
+// (work on another stream, the default one among them, is not ordered before that call's).  A
+// recorded call clears them each time it is replayed; the first one that runs at once, for good.
+struct Tickets {
+    bool clear = false;
+    void use(void* words, size_t count, hipStream_t s) {
+        if (clear) return;
+        plamo::launch_fill_u32(static_cast<uint32_t*>(words), 0, count, s);
+        clear = !capturing(s);
+    }
+};
+
 // Workspace of the split flash prefill for the kernel-level entry, per device, grown on demand
 // (the runtime keeps its own).  Growing synchronises the device before freeing the old one.
 struct FlashWorkspace {
@@ -677,11 +695,12 @@ struct FlashWorkspace {
     float* ml = nullptr;
     uint32_t* tickets = nullptr;
     int tokens = 0;
+    Tickets cleared;
 };
 std::mutex g_flash_ws_mu;
 std::map<int, FlashWorkspace> g_flash_ws;
 
-FlashWorkspace flash_workspace(int tokens) {
+FlashWorkspace flash_workspace(int tokens, hipStream_t s) {
     std::lock_guard<std::mutex> lk(g_flash_ws_mu);
     int dev = 0;
     PLAMO_HIP(hipGetDevice(&dev));
@@ -697,9 +716,9 @@ FlashWorkspace flash_workspace(int tokens) {
         PLAMO_HIP(hipMalloc(&w.o, plamo::flash_part_o_floats(plamo::flash_blocks(tokens)) * 4));
         PLAMO_HIP(hipMalloc(&w.ml, plamo::flash_part_ml_floats(plamo::flash_blocks(tokens)) * 4));
         PLAMO_HIP(hipMalloc(&w.tickets, size_t(plamo::flash_blocks(tokens)) * 4));
-        PLAMO_HIP(hipMemset(w.tickets, 0, size_t(plamo::flash_blocks(tokens)) * 4));
         w.tokens = tokens;
     }
+    w.cleared.use(w.tickets, size_t(plamo::flash_blocks(w.tokens)), s);
     return w;
 }
 
@@ -708,15 +727,10 @@ FlashWorkspace flash_workspace(int tokens) {
 struct AttnWorkspace {
     void* base = nullptr;
     uint32_t parts = 0;
+    Tickets cleared;
 };
 std::mutex g_attn_ws_mu;
 std::map<int, AttnWorkspace> g_attn_ws;
-
-bool capturing(hipStream_t s) {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (s) PLAMO_HIP(hipStreamIsCapturing(s, &status));  // the default stream cannot be captured
-    return status != hipStreamCaptureStatusNone;
-}
 
 // Carves a workspace at `base` (256-byte aligned) into the attention parameter pointers and takes
 // the call's tickets in it.
@@ -735,7 +749,7 @@ void attn_workspace_bind(void* base, uint32_t parts, plamo::AttnParams& a, hipSt
     }
 }
 
-void* attn_workspace(uint32_t parts) {
+void* attn_workspace(uint32_t parts, hipStream_t s) {
     std::lock_guard<std::mutex> lk(g_attn_ws_mu);
     int dev = 0;
     PLAMO_HIP(hipGetDevice(&dev));
@@ -747,9 +761,9 @@ void* attn_workspace(uint32_t parts) {
             w = AttnWorkspace{};
         }
         PLAMO_HIP(hipMalloc(&w.base, plamo::attn_workspace_bytes(parts)));
-        PLAMO_HIP(hipMemset(w.base, 0, size_t(2) * plamo::ATTN_TICKETS * 8));
         w.parts = parts;
     }
+    w.cleared.use(w.base, size_t(plamo::ATTN_TICKETS) * 2, s);
     return w.base;
 }
 
@@ -806,8 +820,9 @@ int plamo_kernel_attention_decode(uint64_t qkv, uint64_t q_norm, uint64_t k_norm
         plamo::AttnParams a{};
         const uint32_t parts = attn_decode_params(qkv, q_norm, k_norm, keys, values, capacity, positions, rows, full,
                                                   local_rope, global_rope, out16, a);
-        attn_workspace_bind(attn_workspace(parts), parts, a, reinterpret_cast<hipStream_t>(stream));
-        attn_decode_launch(a, rows, full != 0, reinterpret_cast<hipStream_t>(stream));
+        const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+        attn_workspace_bind(attn_workspace(parts, s), parts, a, s);
+        attn_decode_launch(a, rows, full != 0, s);
         PLAMO_HIP(hipGetLastError());
     });
 }
@@ -859,7 +874,7 @@ int plamo_kernel_attention_prefill(uint64_t q16, uint64_t keys, uint64_t values,
         f.p0 = uint32_t(p0);
         f.seg = plamo::one_segment(tokens);
         f.full = full ? 1 : 0;
-        const FlashWorkspace ws = flash_workspace(tokens);
+        const FlashWorkspace ws = flash_workspace(tokens, reinterpret_cast<hipStream_t>(stream));
         f.part_o = ws.o;
         f.part_ml = ws.ml;
         f.tickets = ws.tickets;
