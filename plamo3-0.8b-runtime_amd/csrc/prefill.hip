@@ -863,11 +863,18 @@ __device__ __forceinline__ void flash_store(const KvSource& src, const KvStage& 
 }
 
 // Two FP32 values in [0, 1] as BF16 pairs hi + lo (RNE, v_cvt_pk_bf16_f32): hi + lo carries ~16
-// significant bits of each value.  The differences value - hi are exact, so one v_dot2_f32_bf16
-// each (hi times -1 and 0 onto the value) gives the same bits as unpacking hi and subtracting.
-// (The factors stay in registers: as literals the compiler encodes one as the inline constant
-// -1.0, which this instruction does not read as the pair (0, -1).)
+// significant bits of each value.
 __device__ __forceinline__ void split_bf16(float a, float b, uint32_t& hw, uint32_t& lw) {
+    hw = pack_bf16(a, b);
+    lw = pack_bf16(a - lo(hw), b - hi(hw));
+}
+// The same split for the direct kernel, whose vector instructions run beside its products: the
+// differences value - hi are exact, so one v_dot2_f32_bf16 each (hi times -1 and 0 onto the value)
+// gives the same bits in fewer instructions.  (The factors stay in registers: as literals the
+// compiler encodes one as the inline constant -1.0, which this instruction does not read as the
+// pair (0, -1).)  In the staged kernel, which waits for each result, it is the slower one: 500
+// local queries from position 0 32.0 us instead of 30.8.
+__device__ __forceinline__ void split_bf16_dot2(float a, float b, uint32_t& hw, uint32_t& lw) {
     uint32_t first = 0x0000bf80u, second = 0xbf800000u;
     __asm__("" : "+s"(first), "+s"(second));
     hw = pack_bf16(a, b);
@@ -888,12 +895,15 @@ __device__ __forceinline__ void flash_prefill(const FlashParams& pass, const int
     p.keys += size_t(sg.lane) * p.capacity * HEAD_DIM;
     p.values += size_t(sg.lane) * p.capacity * HEAD_DIM;
     if (p.keys_rot) p.keys_rot += size_t(sg.lane) * p.rot_rows * HEAD_DIM;
-    // two key and two value tiles: 16 KB each on the direct path; K rows and V^T, padded, on the
-    // staged one
+    // two key and two value tiles: 16 KB each on the direct path (L); padded K rows and V^T on the
+    // staged one, four arrays that the compiler tells apart (L0 .. L3; parts of one array: 333
+    // local queries from position 3001 45.7 us instead of 45.1)
     constexpr int KT = FK * KST, VT = HEAD_DIM * VST;
-    __shared__ __align__(1024) uint8_t L[DIRECT ? 4 * FK * HEAD_DIM * 2 : 2 * (KT + VT) * 2];
-    uint16_t* const L0 = reinterpret_cast<uint16_t*>(L);
-    uint16_t *const L1 = L0 + KT, *const L2 = L1 + KT, *const L3 = L2 + VT;
+    __shared__ __align__(1024) uint8_t L[DIRECT ? 4 * FK * HEAD_DIM * 2 : 16];
+    __shared__ __align__(1024) uint16_t L0[DIRECT ? 8 : KT];
+    __shared__ __align__(1024) uint16_t L1[DIRECT ? 8 : KT];
+    __shared__ __align__(1024) uint16_t L2[DIRECT ? 8 : VT];
+    __shared__ __align__(1024) uint16_t L3[DIRECT ? 8 : VT];
     __shared__ int s_last;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, half = lane >> 5;
@@ -1252,7 +1262,7 @@ __device__ __forceinline__ void flash_prefill(const FlashParams& pass, const int
                     const float e0 = exp2_det(sc[r][i] - ms), e1 = exp2_det(sc[r][i + 1] - ms);
                     ls += e0;
                     ls += e1;
-                    split_bf16(e0, e1, hw[s & 1][k], lw[s & 1][k]);
+                    split_bf16_dot2(e0, e1, hw[s & 1][k], lw[s & 1][k]);
                 }
                 fence();
             });
