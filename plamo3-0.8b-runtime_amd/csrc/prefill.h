@@ -43,17 +43,26 @@ constexpr int PREFILL_SEGMENTS = MAX_ROWS;
 struct PrefillSegments {
     int n;
     PrefillSegment s[PREFILL_SEGMENTS];
-    // the segment of row t, or of query block b
-    __host__ __device__ int of_token(int t) const {
-        int i = 0;
-        for (int k = 1; k < PREFILL_SEGMENTS; ++k) i = k < n && t >= s[k].token0 ? k : i;
-        return i;
+    // The segment of row t, or of query block b.  Its values are selected, not its index: kernel
+    // arguments read at a computed index are a load that waits for the index.
+    __host__ __device__ PrefillSegment of_token(int t) const {
+        PrefillSegment g = s[0];
+#pragma unroll
+        for (int k = 1; k < PREFILL_SEGMENTS; ++k)
+            if (k < n && t >= s[k].token0) g = s[k];
+        return g;
     }
-    __host__ __device__ int of_block(int b) const {
-        int i = 0;
-        for (int k = 1; k < PREFILL_SEGMENTS; ++k) i = k < n && b >= s[k].first_block ? k : i;
-        return i;
+    __host__ __device__ PrefillSegment of_block(int b) const {
+        PrefillSegment g = s[0];
+#pragma unroll
+        for (int k = 1; k < PREFILL_SEGMENTS; ++k)
+            if (k < n && b >= s[k].first_block) g = s[k];
+        return g;
     }
+    // A single segment is the pass: its rows from 0 on, of the first KV slice.  Kernels then look
+    // nothing up and move no pointer (flash of 3 global queries 8.1 -> 7.9 us, 61 local ones 8.76 ->
+    // 8.67).
+    bool valid() const { return n > 1 || (n == 1 && s[0].token0 == 0 && s[0].first_block == 0 && s[0].lane == 0); }
 };
 
 struct QkPrepParams {

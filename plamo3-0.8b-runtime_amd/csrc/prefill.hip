@@ -668,7 +668,8 @@ __global__ __launch_bounds__(256) void rows_norm_kernel(const RowsNormParams p) 
 __global__ __launch_bounds__(256) void qk_prep_kernel(const QkPrepParams p) {
     const int t = blockIdx.x, tid = threadIdx.x;
     const int hq = tid >> 4, sq = tid & 15;
-    const PrefillSegment sg = p.seg.s[p.seg.of_token(t)];
+    PrefillSegment sg = p.seg.s[0];
+    if (p.seg.n > 1) sg = p.seg.of_token(t);
     const uint32_t ts = uint32_t(t - sg.token0);  // the token within its segment
     const uint32_t pos = p.p0 + ts;
     const uint32_t chunk = p.p0 + (ts / CHUNK) * CHUNK;
@@ -887,14 +888,17 @@ template <bool QSA, bool DIRECT>
 __device__ __forceinline__ void flash_prefill(const FlashParams& pass, const int block, const int part) {
 #pragma clang fp contract(off)  // fixed rounding sequence, reproduced by the CPU oracle
     // block `block` of the pass is block qb of its segment
-    const PrefillSegment sg = pass.seg.s[pass.seg.of_block(block)];
-    const int qb = block - sg.first_block, tokens = sg.tokens;
+    PrefillSegment sg = pass.seg.s[0];
     FlashParams p = pass;
-    p.q += size_t(sg.token0) * ATTN;
-    p.out += size_t(sg.token0) * ATTN;
-    p.keys += size_t(sg.lane) * p.capacity * HEAD_DIM;
-    p.values += size_t(sg.lane) * p.capacity * HEAD_DIM;
-    if (p.keys_rot) p.keys_rot += size_t(sg.lane) * p.rot_rows * HEAD_DIM;
+    if (pass.seg.n > 1) {
+        sg = pass.seg.of_block(block);
+        p.q += size_t(sg.token0) * ATTN;
+        p.out += size_t(sg.token0) * ATTN;
+        p.keys += size_t(sg.lane) * p.capacity * HEAD_DIM;
+        p.values += size_t(sg.lane) * p.capacity * HEAD_DIM;
+        if (p.keys_rot) p.keys_rot += size_t(sg.lane) * p.rot_rows * HEAD_DIM;
+    }
+    const int qb = block - sg.first_block, tokens = sg.tokens;
     // two key and two value tiles: 16 KB each on the direct path (L); padded K rows and V^T on the
     // staged one, four arrays that the compiler tells apart (L0 .. L3; parts of one array: 333
     // local queries from position 3001 45.7 us instead of 45.1)
@@ -1540,6 +1544,7 @@ void launch_gather_last(const uint16_t* a, const uint16_t* b, const PrefillSegme
 
 void launch_qk_prep(const QkPrepParams& p, hipStream_t s) {
     if (p.tokens < 1) return;
+    if (!p.seg.valid()) throw Error(E_INVAL, "prefill: bad segments");
     hipLaunchKernelGGL(qk_prep_kernel, dim3(p.tokens), dim3(256), 0, s, p);
 }
 
@@ -1578,7 +1583,7 @@ void flash_schedule(const FlashParams& p, FlashSchedule& sched) {
         Item items[FLASH_SCHEDULE_MAX];
         int n = 0;
         for (int qb = 0; qb < p.blocks; ++qb) {
-            const PrefillSegment& sg = p.seg.s[p.seg.of_block(qb)];
+            const PrefillSegment sg = p.seg.of_block(qb);
             const int tiles = flash_block_tiles(sg.tokens, p.p0, p.full, qb - sg.first_block), parts = flash_block_parts(tiles);
             for (int q = 0; q < parts; ++q) items[n++] = {(q + 1) * tiles / parts - q * tiles / parts, qb, q};
         }
@@ -1606,6 +1611,7 @@ void flash_schedule(const FlashParams& p, FlashSchedule& sched) {
 
 void launch_flash_prefill(const FlashParams& params, hipStream_t s) {
     FlashParams p = params;
+    if (!p.seg.valid()) throw Error(E_INVAL, "prefill: bad segments");
     p.blocks = flash_blocks(p.seg);
     if (p.blocks < 1) return;
     if (p.blocks > 65536 / FLASH_PARTS) throw Error(E_INVAL, "flash prefill: too many tokens in one call");
