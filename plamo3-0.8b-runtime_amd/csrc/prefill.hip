@@ -1461,7 +1461,9 @@ int gemm_tile(const GemmTile (&tiles)[N], int cols, int tokens, int k) {
         if (t.k256 && k % 256 != 0) continue;
         const int64_t n = int64_t((cols + t.bm - 1) / t.bm) * ((tokens + t.bt - 1) / t.bt);
         const float us = float((n + CUS - 1) / CUS) * t.us;
-        if (best < 0 || us < least) best = int(i), least = us;
+        // of equal times the larger tile, in fewer rounds (qkv of 1,281 to 1,344 tokens: 128 x 128 in
+        // one round 15.6 us, 96 x 64 in two 18.1)
+        if (best < 0 || us <= least) best = int(i), least = us;
     }
     return best;
 }
