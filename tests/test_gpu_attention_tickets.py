@@ -80,6 +80,18 @@ def test_counts_left_in_tickets_change_nothing(full):
         out.zero_()
 
 
+@pytest.mark.parametrize("full", [0, 1])
+@pytest.mark.parametrize("positions", [[513, 476, 130, 127], [511, 512], [1023, 64, 3]])
+def test_rows_together_equal_rows_alone(full, positions):
+    """Which kernel merges a row depends on the rows beside it; its bits do not."""
+    print(f"  positions {positions} full {full}", flush=True)
+    together = _static_call(8, len(positions), positions, full)().clone()
+    for row, pos in enumerate(positions):
+        alone = _static_call(8, len(positions), [pos if q == row else 0 for q in range(len(positions))], full)()
+        torch.cuda.synchronize()
+        assert torch.equal(alone[row], together[row]), row
+
+
 def test_replays_between_calls():
     recorded, other = _static_call(6, 2, [450, 200], 0), _static_call(7, 3, [64, 500, 129], 1)
     want, want_other = recorded().clone(), other().clone()
