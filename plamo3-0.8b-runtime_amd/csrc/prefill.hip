@@ -406,6 +406,12 @@ __device__ __forceinline__ u32x4_t view_words(const void* base, uint32_t bytes) 
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
     return uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p));
 }
+// M0 is reserved (the compiler keeps no value of its own there across a statement), so naming it
+// as clobbered draws a warning at every use; it is named all the same, so that the compiler's own
+// writes of M0 stay in order with these.  (As an input operand in M0 the compiler writes it and no
+// warning comes, but down of 150 tokens takes 11.2 us instead of 11.0.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void load_to_lds_untracked(const u32x4_t view, uint32_t lds, uint32_t off, uint32_t scalar_off = 0) {
     __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                      :
@@ -413,6 +419,7 @@ __device__ __forceinline__ void load_to_lds_untracked(const u32x4_t view, uint32
                        "s"(__builtin_amdgcn_readfirstlane(int(scalar_off)))
                      : "m0", "memory");
 }
+#pragma clang diagnostic pop
 
 // The same product on small tiles, for calls whose 32-row tiles would leave most CUs idle
 // (up to about 1,000 tokens): BT tokens x BM weight rows as 16x16 blocks of
