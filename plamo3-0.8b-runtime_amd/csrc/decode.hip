@@ -941,7 +941,6 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const AttnParams p) {
     __shared__ __align__(16) float ps[HG * KP];
     __shared__ __align__(16) float knew[HEAD_DIM];
     __shared__ float l_s[HG];
-    __shared__ float den_s[HG];
     __shared__ int s_last;
 
     const StepState* st = p.state;
@@ -1235,158 +1234,54 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const AttnParams p) {
     if (!s_last) return;
     const size_t row0 = size_t(q) * p.parts;
     // per head: M = max_p m_p, w_p = exp(m_p - M), den = sum_p l_p w_p (partition order);
-    // then each (h, d) sums o_p w_p in partition order.  Partition statistics are staged in
-    // LDS (the key tile is free now) with all loads in flight together.
-    float* mm = reinterpret_cast<float*>(ks);          // [np][HG]
-    float* wl = mm + (KP * KS) / 2;                    // [np][HG]: l, then the weights
-    const uint32_t np = nparts <= uint32_t(KP * KS / 2 / HG) ? nparts : uint32_t(KP * KS / 2 / HG);
-    // up to 64 partitions one entry per thread; more: eight entries per thread in flight
-    if (np * HG <= 256) {
-        if (uint32_t(tid) < np * HG) {
-            const uint32_t k = uint32_t(tid) / HG, h = hg * HG + uint32_t(tid) % HG;
-            mm[tid] = __uint_as_float(buffer_load4_sc1(mview, uint32_t((row0 + k) * HEADS + h) * 4u));
-            wl[tid] = __uint_as_float(buffer_load4_sc1(lview, uint32_t((row0 + k) * HEADS + h) * 4u));
-        }
-    } else
-    for (uint32_t i0 = tid; i0 < np * HG; i0 += 256 * 8) {
-        float mv[8], lv[8];
-#pragma unroll
-        for (uint32_t j = 0; j < 8; ++j) {
-            const uint32_t i = i0 + 256 * j;
-            if (i < np * HG) {
-                const uint32_t k = i / HG, h = hg * HG + i % HG;
-                mv[j] = __uint_as_float(buffer_load4_sc1(mview, uint32_t((row0 + k) * HEADS + h) * 4u));
-                lv[j] = __uint_as_float(buffer_load4_sc1(lview, uint32_t((row0 + k) * HEADS + h) * 4u));
-            }
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < 8; ++j) {
-            const uint32_t i = i0 + 256 * j;
-            if (i < np * HG) {
-                mm[i] = mv[j];
-                wl[i] = lv[j];
-            }
-        }
+    // then each (h, d) sums o_p w_p in partition order.  At most F partitions (longer rows are
+    // attn_merge_kernel's, launch_attention sees to it): one statistic per thread, staged in LDS
+    // (the key tile is free now), and thread -> dim d = tid & 127 of local heads (tid >> 7) and
+    // (tid >> 7) + 2, its outputs requested together with the statistics.
+    constexpr uint32_t F = ATTN_MERGE_INLINE;
+    static_assert(F * HG <= 256, "one statistic per thread");
+    float* mm = reinterpret_cast<float*>(ks);  // [F][HG]
+    float* wl = mm + F * HG;                   // [F][HG]: l
+    if (uint32_t(tid) < nparts * HG) {
+        const uint32_t k = uint32_t(tid) / HG, h = hg * HG + uint32_t(tid) % HG;
+        mm[tid] = __uint_as_float(buffer_load4_sc1(mview, uint32_t((row0 + k) * HEADS + h) * 4u));
+        wl[tid] = __uint_as_float(buffer_load4_sc1(lview, uint32_t((row0 + k) * HEADS + h) * 4u));
     }
-    // thread -> dim d = tid & 127 of local heads (tid >> 7) and (tid >> 7) + 2.  The outputs
-    // of the first F partitions are requested together with the statistics (only those that
-    // exist); the rest go in chunks of PRE, chunk c + 1 requested while chunk c is summed
-    // (loads past the last partition re-read it, so every chunk issues the same number of
-    // requests and the wait before the sums counts exactly).
     const int d = tid & 127, hb = tid >> 7;
-    constexpr uint32_t F = 8, PRE = 32;
-    float ovf[F][2];
-    auto load_one = [&](uint32_t k, float (&dst)[2]) {
+    float ov[F][2];
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-            dst[i] = __uint_as_float(
-                buffer_load4_sc1(oview, uint32_t(((row0 + k) * HEADS + hg * HG + hb + 2 * i) * HEAD_DIM + d) * 4u));
-    };
-    auto load_chunk = [&](uint32_t c0, float (&dst)[PRE][2]) {
+    for (uint32_t k = 0; k < F; ++k)
+        if (k < nparts) {
 #pragma unroll
-        for (uint32_t j = 0; j < PRE; ++j) load_one(c0 + j < nparts ? c0 + j : nparts - 1, dst[j]);
-    };
-    // Global layers merge only rows of up to F partitions here (every caller hands longer
-    // rows to attn_merge_kernel); a longer one would take the memory path below, which has
-    // the same operations in the same order, so the chunked loop is left out of that kernel.
-    const bool staged = nparts == np && (!FULL || nparts <= F);
-    if (staged) {
-#pragma unroll
-        for (uint32_t j = 0; j < F; ++j)
-            if (j < nparts) load_one(j, ovf[j]);
+            for (int i = 0; i < 2; ++i)
+                ov[k][i] = __uint_as_float(
+                    buffer_load4_sc1(oview, uint32_t(((row0 + k) * HEADS + hg * HG + hb + 2 * i) * HEAD_DIM + d) * 4u));
+        }
+    __syncthreads();
+    // M per head; then every weight exp(m_p - M) in parallel (in place of m_p); then each
+    // thread forms den for its own two heads (partition order) while summing o_p w_p
+    if (tid < HG) {
+        float M = NEG_INF;
+        for (uint32_t k = 0; k < nparts; ++k) M = fmaxf(M, mm[k * HG + tid]);
+        l_s[tid] = M;
     }
     __syncthreads();
-    if (staged) {
-        // M per head; then every weight exp(m_p - M) in parallel (in place of m_p); then each
-        // thread forms den for its own two heads (partition order) while summing o_p w_p
-        // M per head: up to 16 partitions one thread per head; more: wave w takes local head w
-        // (a maximum has no rounding, so any order gives the same M)
-        static_assert(HG == 4, "one wave per local head");
-        if (nparts <= 16) {
-            if (tid < HG) {
-                float M = NEG_INF;
-                for (uint32_t k = 0; k < nparts; ++k) M = fmaxf(M, mm[k * HG + tid]);
-                l_s[tid] = M;
-            }
-        } else {
-            float M = NEG_INF;
-            for (uint32_t k = uint32_t(lane); k < nparts; k += 64) M = fmaxf(M, mm[k * HG + wave]);
-            M = fmaxf(M, xor_lane<32>(M));
-            M = fmaxf(M, xor_lane<16>(M));
-            M = fmaxf(M, xor_lane<8>(M));
-            M = fmaxf(M, xor_lane<4>(M));
-            M = fmaxf(M, xor_lane<2>(M));
-            M = fmaxf(M, xor_lane<1>(M));
-            if (lane == 0) l_s[wave] = M;
+    if (uint32_t(tid) < nparts * HG) mm[tid] = exp_det(mm[tid] - l_s[tid % HG]);
+    __syncthreads();
+    float num[2] = {0.f, 0.f}, den[2] = {0.f, 0.f};
+#pragma unroll
+    for (uint32_t k = 0; k < F; ++k) {
+        if (k >= nparts) break;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const float w = mm[k * HG + hb + 2 * i];
+            num[i] = num[i] + ov[k][i] * w;
+            den[i] = den[i] + wl[k * HG + hb + 2 * i] * w;
         }
-        __syncthreads();
-        for (uint32_t i = tid; i < np * HG; i += 256) mm[i] = exp_det(mm[i] - l_s[i % HG]);
-        __syncthreads();
-        float num[2] = {0.f, 0.f}, den[2] = {0.f, 0.f};
-        float ovp[PRE][2];
-        if constexpr (!FULL)
-            if (F < nparts) load_chunk(F, ovp);
-#pragma unroll
-        for (uint32_t k = 0; k < F; ++k) {
-            if (k >= nparts) break;
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const float w = mm[k * HG + hb + 2 * i];
-                num[i] = num[i] + ovf[k][i] * w;
-                den[i] = den[i] + wl[k * HG + hb + 2 * i] * w;
-            }
-        }
-        for (uint32_t c0 = F; !FULL && c0 < nparts; c0 += PRE) {
-            const bool more = c0 + PRE < nparts;
-            float nxt[PRE][2];
-            if (more) load_chunk(c0 + PRE, nxt);
-#pragma unroll
-            for (uint32_t j = 0; j < PRE; ++j) {
-                const uint32_t k = c0 + j;
-                if (k >= nparts) break;
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const float w = mm[k * HG + hb + 2 * i];
-                    num[i] = num[i] + ovp[j][i] * w;
-                    den[i] = den[i] + wl[k * HG + hb + 2 * i] * w;
-                }
-            }
-            if (more) {
-#pragma unroll
-                for (uint32_t j = 0; j < PRE; ++j) {
-                    ovp[j][0] = nxt[j][0];
-                    ovp[j][1] = nxt[j][1];
-                }
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-            p.out16[size_t(q) * ATTN + (hg * HG + hb + 2 * i) * HEAD_DIM + d] = uint16_t(bits(num[i] / den[i]));
-    } else {  // more partitions than LDS holds (or a global row past F): read them from memory
-        if (tid < HG) {
-            const int h = hg * HG + tid;
-            float M = NEG_INF, den = 0.f;
-            auto pm = [&](uint32_t k) { return __uint_as_float(buffer_load4_sc1(mview, uint32_t((row0 + k) * HEADS + h) * 4u)); };
-            auto pl = [&](uint32_t k) { return __uint_as_float(buffer_load4_sc1(lview, uint32_t((row0 + k) * HEADS + h) * 4u)); };
-            for (uint32_t k = 0; k < nparts; ++k) M = fmaxf(M, pm(k));
-            for (uint32_t k = 0; k < nparts; ++k) den = den + pl(k) * exp_det(pm(k) - M);
-            den_s[tid] = den;
-            l_s[tid] = M;
-        }
-        __syncthreads();
-        float num[2] = {0.f, 0.f};
-        for (uint32_t k = 0; k < nparts; ++k)
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int h = hg * HG + hb + 2 * i;
-                const float ov = __uint_as_float(buffer_load4_sc1(oview, uint32_t(((row0 + k) * HEADS + h) * HEAD_DIM + d) * 4u));
-                const float mk = __uint_as_float(buffer_load4_sc1(mview, uint32_t((row0 + k) * HEADS + h) * 4u));
-                num[i] = num[i] + ov * exp_det(mk - l_s[hb + 2 * i]);
-            }
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-            p.out16[size_t(q) * ATTN + (hg * HG + hb + 2 * i) * HEAD_DIM + d] = uint16_t(bits(num[i] / den_s[hb + 2 * i]));
     }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        p.out16[size_t(q) * ATTN + (hg * HG + hb + 2 * i) * HEAD_DIM + d] = uint16_t(bits(num[i] / den[i]));
     if (tid == 0) atomicExch(ticket, Ticket(0));  // ready for the next launch
 }
 
@@ -1887,6 +1782,8 @@ void launch_gemv(int n, bool packed, int maxr, Prologue pro, Epilogue epi, const
 }
 
 void launch_attention(bool full, const AttnParams& p, int rows, hipStream_t s) {
+    // the attention kernel merges rows of up to ATTN_MERGE_INLINE partitions
+    if ((p.defer ? p.defer : p.parts) > ATTN_MERGE_INLINE) throw Error(E_INVAL, "attention: too many partitions to merge");
     const dim3 grid(32 * ((p.parts + 7) / 8), 1, rows), block(256);
 #define PLAMO_ATTN(F, A) hipLaunchKernelGGL((attn_decode_kernel<F, A>), grid, block, 0, s, p)
     if (p.state) {
