@@ -12,9 +12,11 @@ attention checks, restated for the HIP kernel and computed independently of the 
   count - 1; local rows at 4090.. with a 2064-slot ring; 2050 is the base > 0 case).  Here the
   dense side is an FP32 torch restatement of the same layer (q/k RMSNorm, RoPE, the new key
   and value at pos % capacity, softmax over the visible keys, P.V), and the kernel's BF16
-  output must be within 2e-3 of its unrounded FP32 result.  The 32,768-key rows have 512
-  partitions, merged by attn_merge_kernel; the 4096/8192-key rows go through the in-kernel
-  ticket merge.
+  output must be within 2e-3 of its unrounded FP32 result.  Rows of more than
+  eight partitions of 64 keys are merged by attn_merge_kernel, those of two to eight by the attention
+  kernel's last workgroup.
+The entry point's kernels take positions as arguments.  The runtime's read them from the step state:
+test_gpu_exact.py and test_gpu_long.py compare those with the restatement, bit for bit.
 """
 import ctypes
 
@@ -181,3 +183,9 @@ def test_partitioned_matches_dense_fp32(tables, count, rows, full):
         assert np.array_equal(kc[r, p % cap], bits_np(knew)) and np.array_equal(vc[r, p % cap], bits_np(vnew))
     print(f"    max abs error {worst:.2e}", flush=True)
 
+
+@pytest.mark.parametrize("count,rows,full", [(65, 1, True), (300, 4, True), (512, 1, True), (512, 3, False),
+                                             (449, 1, False), (129, 4, False)])
+def test_merged_in_the_attention_kernel_matches_dense_fp32(tables, count, rows, full):
+    """Two to eight partitions, alone and side by side."""
+    test_partitioned_matches_dense_fp32(tables, count, rows, full)

@@ -10,6 +10,8 @@ the synthetic seed-0 model and random-init indexers (synth.write_auxiliary).
   budget 16, plain and .p12, equal the order-exact CPU twin (oracle/adapters.py QsaTwin on exact.ExactDecoder and
   exact_prefill.ExactPrefill) in every logit bit, the hidden row and the next token, and
   differ from dense attention;
+* the same past 128 keys (a query's second bitmap word), and calls of several hundred tokens whose
+  every block is selected (merged parts, later bitmap words) against dense attention;
 * with MTP: a two-row sequential verification equals two scalar QSA forwards.
 """
 import numpy as np
@@ -151,6 +153,53 @@ def test_prefill_and_decode_bit_exact(model_dir, oracle_weights, packed):
     finally:
         rt.close()
         dense.close()
+
+
+def test_prefill_past_a_bitmap_word_bit_exact(model_dir, oracle_weights):
+    """Keys past 128, whose selected blocks stand in the second word of a query's bitmap: a prompt of
+    137 tokens, then a forward of 13 that starts inside a block."""
+    context, budget = 160, 64
+    prompt = [1] + np.random.default_rng(33).integers(1024, 107520, 149).tolist()
+    adapters = ad.Adapters(model_dir[0])
+    rt = _rt(model_dir, context, budget)
+    try:
+        rt.prefill(prompt[:137])
+        logits, hidden = rt.logit_bits(), rt.hidden().view(np.uint32)
+        nxt = rt.forward(prompt[137:])
+        ex = exact.ExactDecoder(oracle_weights, context, rt.stats()["local_capacity"],
+                                qsa=ad.QsaTwin(adapters, context, budget))
+        pre = xp.ExactPrefill(ex)
+        bits, want, _ = pre.prefill(prompt[:137])
+        print("  137 tokens: the twin is done", flush=True)
+        assert np.array_equal(logits, bits) and np.array_equal(hidden, want.view(np.uint32))
+        bits, want, token = pre.prefill(prompt[137:], p0=137)
+        assert np.array_equal(rt.logit_bits(), bits)
+        assert np.array_equal(rt.hidden().view(np.uint32), want.view(np.uint32))
+        assert nxt == token
+    finally:
+        rt.close()
+
+
+@pytest.mark.parametrize("tokens", [763, 1407])
+def test_every_block_selected_equals_dense(model_dir, tokens):
+    """A budget that every complete block fits, though the call is past it: the QSA kernels, here with
+    query blocks of two and three merged parts and bitmaps of up to eleven words, against dense ones."""
+    budget = tokens // 4 * 4
+    prompt = [1] + np.random.default_rng(tokens).integers(1024, 107520, tokens - 1).tolist()
+    dense, sparse = _rt(model_dir, tokens + 8), _rt(model_dir, tokens + 8, budget)
+    try:
+        print(f"  {tokens} tokens, budget {budget}", flush=True)
+        assert dense.prefill(prompt) == sparse.prefill(prompt)
+        st = sparse.stats()
+        assert st["sparse_queries"] > 0 and st["sparse_keys"] == st["dense_keys"]
+        assert np.array_equal(dense.logit_bits(), sparse.logit_bits())
+        assert np.array_equal(dense.hidden().view(np.uint32), sparse.hidden().view(np.uint32))
+        for layer in (8, 15):  # after the first and the second global layer's attention
+            for a, b in zip(dense.kv(layer), sparse.kv(layer)):
+                assert np.array_equal(a[:tokens], b[:tokens]), layer
+    finally:
+        dense.close()
+        sparse.close()
 
 
 def test_verification_rows_with_qsa(model_dir):
