@@ -31,8 +31,6 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float floatx2 __attribute__((ext_vector_type(2)));
 
 constexpr int BK = 64, LDS_STRIDE = BK + 8;  // +16 B per row against bank conflicts
 
@@ -421,8 +419,9 @@ __device__ __forceinline__ void load_to_lds_untracked(const u32x4_t view, uint32
 }
 #pragma clang diagnostic pop
 
-// The same product on small tiles, for calls whose 32-row tiles would leave most CUs idle
-// (up to about 1,000 tokens): BT tokens x BM weight rows as 16x16 blocks of
+// The same product on tiles of 16x16 blocks, for calls whose tiles of 32-row blocks would leave
+// CUs idle: by gemm_tile's rule every call of up to 960 tokens, and longer ones up to 1,536 (o, down;
+// 96 x 96) or 1,792 (qkv; 128 x 128).  BT tokens x BM weight rows as 16x16 blocks of
 // v_mfma_f32_16x16x32_bf16, whose result equals two v_mfma_f32_32x32x16_bf16 steps bit for bit
 // (both fold K in groups of eight in ascending order), at half the latency per K.  A stage is H
 // slabs of 64 K values, each [BT activation rows | BM weight rows] of 128 bytes loaded and
@@ -962,11 +961,6 @@ __device__ __forceinline__ void flash_prefill(const FlashParams& pass, const int
     // tiles that cross a query's causal edge or window start need the mask.  QSA: every tile
     // is masked by the query's selected blocks (its unfinished block is always seen).  Leaves
     // the probabilities in sacc and rescales oacc.
-    // Online softmax of tile j in the base-2 domain: x = score * scale * log2(e),
-    // p = 2^(x - max).  Element i of tile r is key k0 + 32r + 8(i/4) + 4*half + i%4.  Only
-    // tiles that cross a query's causal edge or window start need the mask.  QSA: every tile
-    // is masked by the query's selected blocks (its unfinished block is always seen).  Leaves
-    // the probabilities in sacc and rescales oacc.
     auto softmax = [&](int j, floatx16 (&sacc)[2]) {
         const uint32_t k0 = klo + uint32_t(j * FK);
         const bool edge = QSA || !(k0 + uint32_t(FK - 1) <= plo && (p.full || k0 + uint32_t(WINDOW - 1) >= khi));
@@ -1448,26 +1442,43 @@ void launch_swiglu_small(const GemmParams& p, hipStream_t s) {
                        cols, rows, wide);
 }
 
+// CUs of the current device.
+int device_cus() {
+    thread_local int of = -1, cus = 0;
+    int device = 0;
+    PLAMO_HIP(hipGetDevice(&device));
+    if (device != of) {
+        PLAMO_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+        cus = std::max(cus, 1);
+        of = device;
+    }
+    return cus;
+}
+
 // A tile of the GEMM kernels and the measured time of one round of it (us; every CU one tile).
 struct GemmTile {
     int bt, bm;
     float us;
     bool k256;  // its stages are 256 deep
 };
-// The tile whose rounds over the CUs take least: rounds = tiles / CUs, rounded up, since the
-// kernels run one workgroup per CU.  A call of few tokens thus takes the largest tiles that
-// still fill the chip, or small ones down to 16 x 16: every CU reads (bt + bm) rows of k values
+// The tile whose rounds over the CUs take least.  A call of few tokens thus takes the largest tiles
+// that still fill the chip, or small ones down to 16 x 16: every CU reads (bt + bm) rows of k values
 // however the tile is cut, so the smallest that fits one round is also the shortest.
+// A round is counted as one tile per CU, and each as long as the first.  That is so for tiles of more
+// than 80 KB of LDS (down at 256 and 512 of them: 64 x 48 21.4 and 41.4 us, 64 x 96 31.2 and 63.6).
+// Of the smaller ones two fit on a CU, and their second round is charged more than it takes: 16 x 16
+// 8.9 and 10.8 us, 16 x 32 11.3 and 14.7, 32 x 32 11.3 and 19.6; gate_up's 16 x 64 8.3 and 9.2, 32 x 64
+// 8.4 and 10.3, 64 x 96 11.3 and 17.1.
 template <size_t N>
 int gemm_tile(const GemmTile (&tiles)[N], int cols, int tokens, int k) {
-    constexpr int CUS = 256;
+    const int cus = device_cus();
     int best = -1;
     float least = 0.f;
     for (size_t i = 0; i < N; ++i) {
         const GemmTile& t = tiles[i];
         if (t.k256 && k % 256 != 0) continue;
         const int64_t n = int64_t((cols + t.bm - 1) / t.bm) * ((tokens + t.bt - 1) / t.bt);
-        const float us = float((n + CUS - 1) / CUS) * t.us;
+        const float us = float((n + cus - 1) / cus) * t.us;
         // of equal times the larger tile, in fewer rounds (qkv of 1,281 to 1,344 tokens: 128 x 128 in
         // one round 15.6 us, 96 x 64 in two 18.1)
         if (best < 0 || us <= least) best = int(i), least = us;
@@ -1586,21 +1597,15 @@ namespace {
 void flash_schedule(const FlashParams& p, FlashSchedule& sched) {
     // the last schedule of local and of global layers, per host thread
     thread_local struct {
-        int device = -1, cus = 0, tokens[PREFILL_SEGMENTS] = {-1};
+        int cus = 0, tokens[PREFILL_SEGMENTS] = {-1};
         uint32_t p0 = 0;
         FlashSchedule sched{};
     } cache[2];
     int lengths[PREFILL_SEGMENTS] = {};
     for (int i = 0; i < p.seg.n; ++i) lengths[i] = p.seg.s[i].tokens;
-    int device = 0;
-    PLAMO_HIP(hipGetDevice(&device));
     auto& c = cache[p.full ? 1 : 0];
-    if (c.device != device) {
-        PLAMO_HIP(hipDeviceGetAttribute(&c.cus, hipDeviceAttributeMultiprocessorCount, device));
-        c.device = device;
-        c.tokens[0] = -1;
-    }
-    if (!std::equal(lengths, lengths + PREFILL_SEGMENTS, c.tokens) || c.p0 != p.p0) {
+    const int C = device_cus();
+    if (c.cus != C || !std::equal(lengths, lengths + PREFILL_SEGMENTS, c.tokens) || c.p0 != p.p0) {
         struct Item {
             int tiles, qb, part;
         };
@@ -1611,7 +1616,6 @@ void flash_schedule(const FlashParams& p, FlashSchedule& sched) {
             const int tiles = flash_block_tiles(sg.tokens, p.p0, p.full, qb - sg.first_block), parts = flash_block_parts(tiles);
             for (int q = 0; q < parts; ++q) items[n++] = {(q + 1) * tiles / parts - q * tiles / parts, qb, q};
         }
-        const int C = std::max(c.cus, 1);
         c.sched.n = 0;
         if (n <= 2 * C) {
             std::sort(items, items + n, [](const Item& a, const Item& b) {
@@ -1627,6 +1631,7 @@ void flash_schedule(const FlashParams& p, FlashSchedule& sched) {
         }
         std::copy(lengths, lengths + PREFILL_SEGMENTS, c.tokens);
         c.p0 = p.p0;
+        c.cus = C;
     }
     sched = c.sched;
 }
