@@ -1282,19 +1282,25 @@ __device__ __forceinline__ void flash_prefill(const FlashParams& pass, const int
         static_for<0, 4>([&](auto t) { request_v(j0, t); });
         tiles_in();
         st_first(0);
-        // A part of one tile (short prompts) has nothing to request or score ahead: with the next
-        // tile's copy requested, waited for and scored all the same, 3 global queries took 8.3 us
-        // instead of 7.3.  (The last tile of longer parts scores a stale copy: an instance of its
-        // own for each buffer left the loop 176 bytes of spilled registers, 500 queries 23.2 -> 29.)
+        // A part of one tile (short prompts) has nothing to request or score ahead, nor has the
+        // second of two: with a stale copy requested, waited for and scored all the same, 3 global
+        // queries took 8.3 us instead of 7.3, 100 queries 10.1 instead of 9.8.  The last tile of
+        // longer parts does score one: an instance without in their loop costs it more in spilled
+        // registers (500 queries 23.1 -> 26 to 29 us).
         if (j0 + 1 < j1) static_for<0, 4>([&](auto t) { request_k(j0 + 1, t); });
         static_for<0, 16>([&](auto n) { st(0, n, sa); });
         if (j0 + 1 < j1) {
-            int j = j0;
-            do {
-                tile(j, std::integral_constant<int, 0>{}, std::true_type{}, sa, sb);
-                if (j + 1 < j1) tile(j + 1, std::integral_constant<int, 1>{}, std::true_type{}, sb, sa);
-                j += 2;
-            } while (j < j1);
+            if (j0 + 2 < j1) {
+                int j = j0;
+                do {
+                    tile(j, std::integral_constant<int, 0>{}, std::true_type{}, sa, sb);
+                    if (j + 1 < j1) tile(j + 1, std::integral_constant<int, 1>{}, std::true_type{}, sb, sa);
+                    j += 2;
+                } while (j < j1);
+            } else {
+                tile(j0, std::integral_constant<int, 0>{}, std::true_type{}, sa, sb);
+                tile(j0 + 1, std::integral_constant<int, 1>{}, std::false_type{}, sb, sa);
+            }
         } else {
             tile(j0, std::integral_constant<int, 0>{}, std::false_type{}, sa, sb);
         }
