@@ -674,9 +674,15 @@ __global__ __launch_bounds__(256) void rows_norm_kernel(const RowsNormParams p) 
 __global__ __launch_bounds__(256) void qk_prep_kernel(const QkPrepParams p) {
     const int t = blockIdx.x, tid = threadIdx.x;
     const int hq = tid >> 4, sq = tid & 15;
-    PrefillSegment sg = p.seg.s[0];
-    if (p.seg.n > 1) sg = p.seg.of_token(t);
-    const uint32_t ts = uint32_t(t - sg.token0);  // the token within its segment
+    uint32_t ts = uint32_t(t);  // the token within its segment
+    uint16_t *keys = p.keys, *values = p.values, *keys_rot = p.keys_rot;
+    if (p.seg.n > 1) {
+        const PrefillSegment sg = p.seg.of_token(t);
+        ts -= uint32_t(sg.token0);
+        keys += size_t(sg.lane) * p.capacity * HEAD_DIM;
+        values += size_t(sg.lane) * p.capacity * HEAD_DIM;
+        if (keys_rot) keys_rot += size_t(sg.lane) * p.rot_rows * HEAD_DIM;
+    }
     const uint32_t pos = p.p0 + ts;
     const uint32_t chunk = p.p0 + (ts / CHUNK) * CHUNK;
     const uint32_t base = chunk > uint32_t(WINDOW - 1) ? chunk - uint32_t(WINDOW - 1) : 0u;
@@ -689,7 +695,7 @@ __global__ __launch_bounds__(256) void qk_prep_kernel(const QkPrepParams p) {
     };
     // the key part's inputs (threads 0..15) are requested with the queries'
     const bool kthread = tid < 16;
-    const bool krot = !p.full && p.keys_rot && pos < p.rot_rows;
+    const bool krot = !p.full && keys_rot && pos < p.rot_rows;
     float4 klo = make_float4(0.f, 0.f, 0.f, 0.f), khi = klo;
     uint2 kgl = make_uint2(0, 0), kgh = kgl;
     uint4 kr4 = make_uint4(0, 0, 0, 0);
@@ -717,7 +723,7 @@ __global__ __launch_bounds__(256) void qk_prep_kernel(const QkPrepParams p) {
         *reinterpret_cast<uint2*>(qo + sq * 4) = make_uint2(pack_bf16(z[0], z[1]), pack_bf16(z[2], z[3]));
         *reinterpret_cast<uint2*>(qo + 64 + sq * 4) = make_uint2(pack_bf16(z[4], z[5]), pack_bf16(z[6], z[7]));
     }
-    const size_t slot = (size_t(sg.lane) * p.capacity + pos % p.capacity) * HEAD_DIM;
+    const size_t slot = size_t(pos % p.capacity) * HEAD_DIM;
     if (kthread) {
         float z[8];
         head_norm8(klo, khi, kgl, kgh, z);
@@ -730,17 +736,17 @@ __global__ __launch_bounds__(256) void qk_prep_kernel(const QkPrepParams p) {
             float zr[8] = {z[0], z[1], z[2], z[3], z[4], z[5], z[6], z[7]};
 #pragma unroll
             for (int j = 0; j < 4; j += 2) rope_pair_x2f(zr[j], zr[4 + j], c4[j], zr[j + 1], zr[4 + j + 1], c4[j + 1]);
-            uint16_t* kr = p.keys_rot + (size_t(sg.lane) * p.rot_rows + pos) * HEAD_DIM;
+            uint16_t* kr = keys_rot + size_t(pos) * HEAD_DIM;
             *reinterpret_cast<uint2*>(kr + tid * 4) = make_uint2(pack_bf16(zr[0], zr[1]), pack_bf16(zr[2], zr[3]));
             *reinterpret_cast<uint2*>(kr + 64 + tid * 4) = make_uint2(pack_bf16(zr[4], zr[5]), pack_bf16(zr[6], zr[7]));
         }
         auto word = [](float a, float b) { return (bits(a) & 0xffffu) | (bits(b) << 16); };
-        *reinterpret_cast<uint2*>(p.keys + slot + tid * 4) = make_uint2(word(z[0], z[1]), word(z[2], z[3]));
-        *reinterpret_cast<uint2*>(p.keys + slot + 64 + tid * 4) = make_uint2(word(z[4], z[5]), word(z[6], z[7]));
+        *reinterpret_cast<uint2*>(keys + slot + tid * 4) = make_uint2(word(z[0], z[1]), word(z[2], z[3]));
+        *reinterpret_cast<uint2*>(keys + slot + 64 + tid * 4) = make_uint2(word(z[4], z[5]), word(z[6], z[7]));
     }
     if (tid >= 64 && tid < 64 + HEAD_DIM) {
         const int d = tid - 64;
-        p.values[slot + d] = x[ATTN + HEAD_DIM + d];
+        values[slot + d] = x[ATTN + HEAD_DIM + d];
     }
 }
 
