@@ -895,8 +895,12 @@ __device__ __forceinline__ void split_bf16_dot2(float a, float b, uint32_t& hw, 
 }
 
 // Part `part` of query block qb.  QSA: global layers with a selection bitmap (a separate
-// instance, so the dense kernel's edge tiles carry no bitmap test).
-template <bool QSA, bool DIRECT>
+// instance, so the dense kernel's edge tiles carry no bitmap test).  SHORT: no block of the call
+// has more than two tiles, and the last requests and scores nothing ahead.  In the longer calls'
+// kernel a stale copy is requested, waited for and scored there: 3 global queries take 8.3 us in it
+// and 7.0 in this one, 100 10.1 and 9.2.  (Both in one kernel cost its loop up to 260 bytes of
+// spilled registers and 500 queries up to 29 us instead of 23.)
+template <bool QSA, bool DIRECT, bool SHORT>
 __device__ __forceinline__ void flash_prefill(const FlashParams& pass, const int block, const int part) {
 #pragma clang fp contract(off)  // fixed rounding sequence, reproduced by the CPU oracle
     // block `block` of the pass is block qb of its segment
@@ -1179,7 +1183,7 @@ __device__ __forceinline__ void flash_prefill(const FlashParams& pass, const int
         auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
 
         // Tile j (buffer B), whose scores are in sc; with NEXT the scores of tile j + 1 go to sn
-        // (after the last tile of several: of stale keys, for nobody)
+        // (without SHORT, after the last tile: of stale keys, for nobody)
         auto tile = [&](int j, auto par, auto next, floatx16 (&sc)[2], floatx16 (&sn)[2]) {
             constexpr int B = decltype(par)::value;
             constexpr bool NEXT = decltype(next)::value;
@@ -1288,25 +1292,16 @@ __device__ __forceinline__ void flash_prefill(const FlashParams& pass, const int
         static_for<0, 4>([&](auto t) { request_v(j0, t); });
         tiles_in();
         st_first(0);
-        // A part of one tile (short prompts) has nothing to request or score ahead, nor has the
-        // second of two: with a stale copy requested, waited for and scored all the same, 3 global
-        // queries took 8.3 us instead of 7.3, 100 queries 10.1 instead of 9.8.  The last tile of
-        // longer parts does score one: an instance without in their loop costs it more in spilled
-        // registers (500 queries 23.1 -> 26 to 29 us).
-        if (j0 + 1 < j1) static_for<0, 4>([&](auto t) { request_k(j0 + 1, t); });
+        if (!SHORT || j0 + 1 < j1) static_for<0, 4>([&](auto t) { request_k(j0 + 1, t); });
         static_for<0, 16>([&](auto n) { st(0, n, sa); });
-        if (j0 + 1 < j1) {
-            if (j0 + 2 < j1) {
-                int j = j0;
-                do {
-                    tile(j, std::integral_constant<int, 0>{}, std::true_type{}, sa, sb);
-                    if (j + 1 < j1) tile(j + 1, std::integral_constant<int, 1>{}, std::true_type{}, sb, sa);
-                    j += 2;
-                } while (j < j1);
-            } else {
-                tile(j0, std::integral_constant<int, 0>{}, std::true_type{}, sa, sb);
-                tile(j0 + 1, std::integral_constant<int, 1>{}, std::false_type{}, sb, sa);
+        if constexpr (!SHORT) {
+            for (int j = j0; j < j1; j += 2) {
+                tile(j, std::integral_constant<int, 0>{}, std::true_type{}, sa, sb);
+                if (j + 1 < j1) tile(j + 1, std::integral_constant<int, 1>{}, std::true_type{}, sb, sa);
             }
+        } else if (j0 + 1 < j1) {
+            tile(j0, std::integral_constant<int, 0>{}, std::true_type{}, sa, sb);
+            tile(j0 + 1, std::integral_constant<int, 1>{}, std::false_type{}, sb, sa);
         } else {
             tile(j0, std::integral_constant<int, 0>{}, std::false_type{}, sa, sb);
         }
@@ -1314,7 +1309,7 @@ __device__ __forceinline__ void flash_prefill(const FlashParams& pass, const int
     }
     // O = O^T / l; element i of d-tile dt is dim 32dt + 8(i/4) + 4*half + i%4
     float lt = ls + xor_lane<32>(ls);
-    if (parts > 1) {
+    if (!SHORT && parts > 1) {
         // Partial (m, l, unnormalised O^T) of this part; the last part to finish merges all
         // parts of the block in part order: M = max m_q, w_q = 2^(m_q - M),
         // O = sum O_q w_q / sum l_q w_q.  A lane writes its sixteen 16-byte pieces where the same
@@ -1398,17 +1393,17 @@ __device__ __forceinline__ void flash_prefill(const FlashParams& pass, const int
 // Workgroup w takes part w / blocks of query block blocks - 1 - w % blocks (consecutive
 // workgroups, dealt round-robin to the XCDs, take different blocks; a block's parts share an
 // XCD) and returns if the block has fewer parts.
-template <bool QSA, bool DIRECT>
+template <bool QSA, bool DIRECT, bool SHORT>
 __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const FlashParams p) {
     const int nqb = p.blocks;
-    flash_prefill<QSA, DIRECT>(p, nqb - 1 - int(blockIdx.x) % nqb, int(blockIdx.x) / nqb);
+    flash_prefill<QSA, DIRECT, SHORT>(p, nqb - 1 - int(blockIdx.x) % nqb, int(blockIdx.x) / nqb);
 }
 
 // Workgroup w takes the item the host's schedule ranks for it (qb << 2 | part).
 template <bool QSA, bool DIRECT>
 __global__ __launch_bounds__(256, 2) void flash_prefill_ranked_kernel(const FlashParams p, const FlashSchedule sched) {
     const uint32_t item = sched.item[blockIdx.x];
-    flash_prefill<QSA, DIRECT>(p, int(item >> 2), int(item & 3u));
+    flash_prefill<QSA, DIRECT, false>(p, int(item >> 2), int(item & 3u));
 }
 
 template <int BT, int BW, int WT, int NT, int NS>
@@ -1657,9 +1652,6 @@ void launch_flash_prefill(const FlashParams& params, hipStream_t s) {
     if (p.blocks < 1) return;
     if (p.blocks > 65536 / FLASH_PARTS) throw Error(E_INVAL, "flash prefill: too many tokens in one call");
     const bool qsa = p.full && p.qsa_mask;
-    FlashSchedule sched;
-    sched.n = 0;
-    if (p.blocks * FLASH_PARTS <= FLASH_SCHEDULE_MAX) flash_schedule(p, sched);
     // keys straight into LDS when no block of the call rotates its keys: global layers, and
     // local layers whose keys all sit in the rotated-key cache (window base 0)
     uint32_t last = 0;
@@ -1667,6 +1659,16 @@ void launch_flash_prefill(const FlashParams& params, hipStream_t s) {
     const bool direct = p.capacity >= uint32_t(FK) &&
                         (p.full || (p.keys_rot != nullptr && last < p.rot_rows && last < uint32_t(WINDOW)));
     const dim3 block(256);
+    // every block within two tiles of keys (key `last` is the last of them): one part each
+    if (direct && last < uint32_t(2 * FK)) {
+        const dim3 grid(uint32_t(p.blocks));
+        if (qsa) hipLaunchKernelGGL((flash_prefill_kernel<true, true, true>), grid, block, 0, s, p);
+        else hipLaunchKernelGGL((flash_prefill_kernel<false, true, true>), grid, block, 0, s, p);
+        return;
+    }
+    FlashSchedule sched;
+    sched.n = 0;
+    if (p.blocks * FLASH_PARTS <= FLASH_SCHEDULE_MAX) flash_schedule(p, sched);
     if (sched.n) {
         // the schedule travels in the kernel arguments (1.5 KB): only the launches that use it
         const dim3 grid(sched.n);
@@ -1677,7 +1679,7 @@ void launch_flash_prefill(const FlashParams& params, hipStream_t s) {
 #undef PLAMO_FLASH
     } else {
         const dim3 grid(uint32_t(p.blocks * FLASH_PARTS));
-#define PLAMO_FLASH(Q, D) hipLaunchKernelGGL((flash_prefill_kernel<Q, D>), grid, block, 0, s, p)
+#define PLAMO_FLASH(Q, D) hipLaunchKernelGGL((flash_prefill_kernel<Q, D, false>), grid, block, 0, s, p)
         if (qsa) PLAMO_FLASH(true, true);
         else if (direct) PLAMO_FLASH(false, true);
         else PLAMO_FLASH(false, false);

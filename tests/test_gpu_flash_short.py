@@ -1,6 +1,6 @@
-"""Global prefill attention at the edge between one key tile and two (a part of one tile has a path of
-its own in the direct kernel), and at the smallest ring that the direct kernel takes and the largest
-that it leaves to the staged one: bit for bit the CPU restatement."""
+"""Global prefill attention at the edges between one key tile, two (calls of up to two have a kernel of
+their own) and three, and at the smallest ring that the direct kernel takes and the largest that it
+leaves to the staged one: bit for bit the CPU restatement."""
 import numpy as np
 import pytest
 import torch
@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("p0,tokens,cap", [
     (0, 1, 64), (0, 63, 64), (3, 61, 64), (63, 1, 64),     # one tile, a partial one and a full one
     (3, 62, 65), (64, 1, 65), (60, 9, 80),                 # blocks of one tile and of two in one call
-    (0, 128, 128), (127, 2, 200),                          # two full tiles, and three
+    (0, 128, 128), (120, 8, 128),                          # two full tiles: the last call of the short kernel
+    (127, 2, 200), (0, 129, 129),                          # three: the first of the other
     (10, 53, 63),                                          # a ring below one tile
 ])
 def test_short_global_calls_bit_exact(p0, tokens, cap):
