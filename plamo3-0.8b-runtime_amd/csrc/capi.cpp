@@ -1,5 +1,6 @@
 // extern "C" boundary (include/plamo_hip.h).  No C++ exception crosses it.
 #include <atomic>
+#include <algorithm>
 #include <chrono>
 #include <cstdio>
 #include <cstring>
@@ -676,8 +677,8 @@ bool capturing(hipStream_t s) {
     return status != hipStreamCaptureStatusNone;
 }
 
-// Tickets of a workspace that has just grown are cleared on the stream of the call that uses them
-// (work on another stream, the default one among them, is not ordered before that call's).  A
+// Tickets of a workspace that has just grown are cleared on the stream of the first call that uses
+// them (work on another stream, the default one among them, is not ordered before that call's).  A
 // recorded call clears them each time it is replayed; the first one that runs at once, for good.
 struct Tickets {
     bool clear = false;
@@ -763,7 +764,7 @@ void* attn_workspace(uint32_t parts, hipStream_t s) {
         PLAMO_HIP(hipMalloc(&w.base, plamo::attn_workspace_bytes(parts)));
         w.parts = parts;
     }
-    w.cleared.use(w.base, size_t(plamo::ATTN_TICKETS) * 2, s);
+    if (parts > 1) w.cleared.use(w.base, size_t(plamo::ATTN_TICKETS) * 2, s);
     return w.base;
 }
 
@@ -877,11 +878,19 @@ int plamo_kernel_attention_prefill(uint64_t q16, uint64_t keys, uint64_t values,
         f.p0 = uint32_t(p0);
         f.seg = plamo::one_segment(tokens);
         f.full = full ? 1 : 0;
-        const FlashWorkspace ws = flash_workspace(tokens, reinterpret_cast<hipStream_t>(stream));
-        f.part_o = ws.o;
-        f.part_ml = ws.ml;
-        f.tickets = ws.tickets;
-        plamo::launch_flash_prefill(f, reinterpret_cast<hipStream_t>(stream));
+        const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+        // the workspace for calls with blocks of several parts (the last full block has the most tiles)
+        const int blocks = plamo::flash_blocks(tokens);
+        int tiles = 0;
+        for (int qb = std::max(0, blocks - 2); qb < blocks; ++qb)
+            tiles = std::max(tiles, plamo::flash_block_tiles(tokens, f.p0, f.full, qb));
+        if (plamo::flash_block_parts(tiles) > 1) {
+            const FlashWorkspace ws = flash_workspace(tokens, s);
+            f.part_o = ws.o;
+            f.part_ml = ws.ml;
+            f.tickets = ws.tickets;
+        }
+        plamo::launch_flash_prefill(f, s);
         PLAMO_HIP(hipGetLastError());
     });
 }

@@ -1,6 +1,7 @@
 """Global prefill attention at the edges between one key tile, two (calls of up to two have a kernel of
 their own) and three, and at the smallest ring that the direct kernel takes and the largest that it
-leaves to the staged one: bit for bit the CPU restatement."""
+leaves to the staged one; and at the edge between blocks of one part and of two, from where a call uses
+the shared workspace: bit for bit the CPU restatement."""
 import numpy as np
 import pytest
 import torch
@@ -18,6 +19,7 @@ pytestmark = pytest.mark.gpu
     (0, 128, 128), (120, 8, 128),                          # two full tiles: the last call of the short kernel
     (127, 2, 200), (0, 129, 129),                          # three: the first of the other
     (10, 53, 63),                                          # a ring below one tile
+    (696, 8, 704), (697, 8, 705), (696, 9, 705),           # one part, two, and both in one call
 ])
 def test_short_global_calls_bit_exact(p0, tokens, cap):
     print(f"  flash p0={p0} tokens={tokens} cap={cap}", flush=True)
